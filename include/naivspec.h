@@ -87,6 +87,40 @@ int nsv_verify_attention(void* out, const void* q, const void* k_cache,
                          size_t workspace_bytes, void* stream);
 
 /*
+ * Causal prefill attention (bf16): rows of several prompts attend keys 0 ..
+ * their position.
+ * Replaces layers/attention.py:123-363 (the varlen and the paged prefill
+ * attention).  The rows are given as tiles, 8 int32 words each:
+ *   [sequence, first row of q/out, rows (1 .. tile_rows), position of the
+ *    first row, first K/V row (contiguous K/V), first key (a multiple of
+ *    64), end key, slot]
+ * A tile's row r attends the keys j <= position + r of its sequence with
+ * first key <= j < end key.  slot -1: those are all its keys and the tile is
+ * written to out.  Slot s >= 0: the tile is cut over keys into several
+ * records with consecutive slots, each written to partials
+ * ([slots, H, tile_rows, D + 2] fp32), and a merge record
+ *   [first slot, records, first row of out, rows]
+ * combines them in a second kernel.
+ *   q, out  [rows, H, D]
+ *   k, v    block_tables == NULL: [keys, Hkv, D], key j of a tile's sequence
+ *           at row tile[4] + j; else paged [num_blocks, block_size, Hkv, D],
+ *           key j in page block_tables[tile[0], j / block_size] (a key whose
+ *           page is negative is not attended; keys past max_blocks *
+ *           block_size do not exist)
+ *   tiles   [ntiles, 8], merges [nmerges, 4] int32, device memory; heavier
+ *           tiles first fill the chip best
+ * Supported: D in {64, 128}; H % Hkv == 0; tile_rows 64 or 128 when H / Hkv
+ * is even, 128 or 256 otherwise; block_size a power of two, a record's keys
+ * on at most 2048 pages.
+ */
+int nsv_prefill_attention(void* out, const void* q, const void* k,
+                          const void* v, const int32_t* block_tables,
+                          const int32_t* tiles, int ntiles, int tile_rows,
+                          const int32_t* merges, int nmerges, float scale,
+                          int H, int Hkv, int D, int block_size,
+                          int max_blocks, void* partials, void* stream);
+
+/*
  * Load-only measurement kernels, no reference counterpart (the ceilings
  * against which bench.py --ceiling reads the verify-attention kernels).
  * nsv_verify_attention_load_floor reads exactly the K/V bytes of a bf16,

@@ -1,0 +1,422 @@
+// Causal prefill attention for gfx950 (bf16): every new row of a prompt
+// attends keys 0 .. its position, from the paged cache (a prompt behind a
+// cached prefix) or from the step's own contiguous K/V.
+//
+// Behaviour follows the reference's prefill attention
+// (src/myvllm/layers/attention.py:123-363: the varlen path over contiguous
+// K/V and the paged path behind a cached prefix); the kernel is this
+// library's own.
+//
+// What bounds it: two matrix products of 4 D flops per (row, key) pair,
+// against one exponential per pair (a quarter-rate VALU operation, about as
+// long as the pair's products).  The host cuts the rows of all sequences
+// into tiles (heaviest first); a workgroup takes one tile of rows for HW
+// query heads of one kv head, so its K/V tiles, staged once in LDS, serve
+// HW heads.  A wave holds 32 rows: S^T = K Q^T on v_mfma_f32_32x32x16_bf16
+// puts a row's scores into two lanes' registers (the row maximum is a
+// register tree and one permlane swap), and its result layout is the B
+// operand of O^T = V^T P^T, V^T coming from the transposing LDS reads.  The
+// workgroup ids of one kv head agree mod 8 at 8 kv heads, so a head's K/V
+// stays in one XCD's L2.
+//
+// Measured on MI355X (the verify kernel on causal blocks of 64 / G rows,
+// which every prefill ran on before -> this kernel): 8 prompts of ~1000
+// tokens, 16/8 heads, 538 -> 59 us (557 TFLOP/s); prompts of 2900 and 4050
+// tokens behind 4096 cached keys, 32/8 heads, 5283 -> 781 us (858); 8192
+// tokens, 32/8 heads, 590 us (932); one prompt of 1206 tokens, 16/8 heads,
+// 85 -> 31 us.
+
+#include "common.h"
+
+namespace {
+
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef short i16x4 __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) i16x4 lds_i16x4;
+
+constexpr int kKeys = 64;          // keys per tile
+constexpr int kWaveRows = 32;      // query rows per wave
+constexpr int kMaxPages = 2048;    // block-table entries staged in LDS
+constexpr int kTileWords = 8;      // int32 words of a tile record
+constexpr float kNegInf = -__builtin_inff();
+// how far (log2 domain) a row's maximum may pass its exponent reference
+// before the reference moves (weights stay <= 2^8, far inside fp32)
+constexpr float kRefSlack = 8.f;
+
+struct PrefillArgs {
+  const bf16_t* q;
+  const bf16_t* k;
+  const bf16_t* v;
+  bf16_t* out;
+  const int32_t* block_tables;  // null: contiguous K/V
+  const int32_t* tiles;         // [ntiles][kTileWords]: sequence, first row, rows, first position, first K/V row,
+                                // first key, end key, partial slot (-1: the tile's only part)
+  float* part;                  // [slots][H][tile_rows][DH + 2]: unnormalised rows, then (max, sum) pairs
+  int tile_rows;
+  float scale_log2;
+  int H, Hkv, bs_log2, max_blocks;
+  int hw;                       // query heads of a kv head one workgroup serves
+  int hgroups;                  // workgroups per (tile, kv head): (H / Hkv) / hw
+};
+
+__device__ __forceinline__ bf16x8 as_bf16x8(u32x4 v) { return __builtin_bit_cast(bf16x8, v); }
+
+__device__ __forceinline__ uint2 lds_read_tr(const unsigned char* p) {
+  const i16x4 v = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*)(p));
+  return __builtin_bit_cast(uint2, v);
+}
+
+// the other half-wave's value of the same row (lane ^ 32) combined
+__device__ __forceinline__ float half_max(float v) {
+  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+__device__ __forceinline__ float half_sum(float v) {
+  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+
+template <int DH, int NW>
+__global__ __launch_bounds__(NW * 64, 2) void prefill_attn_kernel(PrefillArgs a) {
+  constexpr int NT = NW * 64;
+  constexpr int CPR = DH / 8;              // 16-byte chunks per row
+  constexpr int ROWB = DH * 2;             // bytes per staged row
+  constexpr int KS = DH / 16;              // k-steps of S^T
+  constexpr int DT = DH / 32;              // 32-dim tiles of O^T
+  constexpr int LD = kKeys * CPR / NT;     // 16-byte K (and V) loads per thread and tile
+  constexpr int TILEB = kKeys * ROWB;
+  static_assert(LD >= 1 && kKeys * CPR % NT == 0, "whole tiles per pass");
+  struct __attribute__((aligned(16))) Lds {
+    int pages[kMaxPages];
+    int holes;
+    __attribute__((aligned(16))) unsigned char kt[2][TILEB];
+    __attribute__((aligned(16))) unsigned char vt[2][TILEB];
+  };
+  __shared__ Lds lds;
+
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int col = lane & 31, h = lane >> 5;
+  // workgroup -> (tile, head group, kv head), the kv head fastest
+  const int hk = blockIdx.x % a.Hkv;
+  const int rest = blockIdx.x / a.Hkv;
+  const int hg = rest % a.hgroups;
+  const int32_t* rec = a.tiles + (int64_t)(rest / a.hgroups) * kTileWords;
+  const int seq = rec[0], row0 = rec[1], nrows = rec[2], pos0 = rec[3], kv0 = rec[4];
+  const int key_begin = rec[5], slot = rec[7];
+  const int wph = NW / a.hw;               // waves per head
+  const int head = hk * (a.H / a.Hkv) + hg * a.hw + w / wph;
+  const int r0 = (w % wph) * kWaveRows;    // this wave's first row in the tile
+  const bool paged = a.block_tables != nullptr;
+  const int bs_mask = (1 << a.bs_log2) - 1;
+  int key_end = min(rec[6], pos0 + nrows);  // (keys past the tile's last row are never attended)
+  if (paged)  // the table's width, and the staged pages
+    key_end = min(key_end, min(a.max_blocks, (key_begin >> a.bs_log2) + kMaxPages) << a.bs_log2);
+  const int64_t tok = (int64_t)a.Hkv * DH; // elements between consecutive keys
+
+  // query rows as the B operand of S^T: lane (h, col) holds row col, dims 16 ks + 8 h .. + 7
+  bf16x8 qB[KS];
+  {
+    const int r = min(r0 + col, nrows - 1);  // rows past the tile's last load it and are not stored
+    const bf16_t* src = a.q + ((int64_t)(row0 + r) * a.H + head) * DH + h * 8;
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) qB[ks] = as_bf16x8(*reinterpret_cast<const u32x4*>(src + ks * 16));
+  }
+  const int pos = pos0 + r0 + col;           // position of this lane's row
+  const int pos_first = pos0 + r0;           // of the wave's first row
+  const int pos_last = min(pos_first + kWaveRows - 1, pos0 + nrows - 1);
+
+  const int pg0 = key_begin >> a.bs_log2;    // first page staged
+  if (paged) {
+    if (tid == 0) lds.holes = 0;
+    __syncthreads();
+    const int npg = ((key_end + bs_mask) >> a.bs_log2) - pg0;
+    const int32_t* bt = a.block_tables + (int64_t)seq * a.max_blocks + pg0;
+    for (int i = tid; i < npg; i += NT) {
+      const int p = bt[i];
+      lds.pages[i] = p;
+      if (p < 0) lds.holes = 1;
+    }
+    __syncthreads();
+  }
+  const bool holes = paged && __builtin_amdgcn_readfirstlane(lds.holes) != 0;
+
+  // K/V rows of a tile: thread -> rows tid / CPR + j NT / CPR, chunk tid % CPR
+  const int lr = tid / CPR, lc = tid % CPR;
+  u32x4 kr[LD], vr[LD];
+  auto issue = [&](int n0) {
+#pragma unroll
+    for (int j = 0; j < LD; ++j) {
+      const int key = n0 + lr + j * (NT / CPR);
+      const int kc = min(key, key_end - 1);
+      int64_t row = kv0 + kc;
+      if (paged) row = ((int64_t)max(lds.pages[(kc >> a.bs_log2) - pg0], 0) << a.bs_log2) + (kc & bs_mask);
+      const int64_t off = row * tok + hk * DH + lc * 8;
+      kr[j] = *reinterpret_cast<const u32x4*>(a.k + off);
+      vr[j] = *reinterpret_cast<const u32x4*>(a.v + off);
+    }
+  };
+  // K chunk X of key r at slot X ^ (r % CPR); V chunk X at X ^ 4 (r % 4): the
+  // operand reads of a half-wave then touch every bank once
+  auto vswz = [](int r) { return ((r & 3) << 2) & (CPR - 1); };
+  auto stage = [&](int buf, int n0) {
+#pragma unroll
+    for (int j = 0; j < LD; ++j) {
+      const int r = lr + j * (NT / CPR);
+      const int key = n0 + r;
+      bool ok = key < key_end;
+      if (holes && ok) ok = lds.pages[(key >> a.bs_log2) - pg0] >= 0;
+      const u32x4 zero = {0u, 0u, 0u, 0u};
+      *reinterpret_cast<u32x4*>(&lds.kt[buf][r * ROWB + ((lc ^ (r & (CPR - 1))) << 4)]) = ok ? kr[j] : zero;
+      *reinterpret_cast<u32x4*>(&lds.vt[buf][r * ROWB + ((lc ^ vswz(r)) << 4)]) = ok ? vr[j] : zero;
+    }
+  };
+
+  f32x16 acc[DT];
+#pragma unroll
+  for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) acc[dt][i] = 0.f;
+  float m_ref = kNegInf, l_run = 0.f;
+  const float sc = a.scale_log2;
+
+  auto compute = [&](int buf, int n0) {
+    if (n0 > pos_last) return;  // uniform: every key lies past this wave's rows
+    const unsigned char* kt = lds.kt[buf];
+    const unsigned char* vt = lds.vt[buf];
+    f32x16 s[2];
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) s[t][i] = 0.f;
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) {
+        const int r = t * 32 + col;
+        const u32x4 ka = *reinterpret_cast<const u32x4*>(kt + r * ROWB + (((ks * 2 + h) ^ (r & (CPR - 1))) << 4));
+        s[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_bf16x8(ka), qB[ks], s[t], 0, 0, 0);
+      }
+    // lane (h, col), element i of tile t: key n0 + 32 t + 8 (i / 4) + 4 h + i % 4, row col
+    if (n0 + kKeys - 1 > pos_first || holes) {
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+          const int key = n0 + t * 32 + (i >> 2) * 8 + h * 4 + (i & 3);
+          bool ok = key <= pos;
+          if (holes) ok = ok && lds.pages[(min(key, key_end - 1) >> a.bs_log2) - pg0] >= 0;
+          s[t][i] = ok ? s[t][i] : kNegInf;
+        }
+    }
+    float mx = fmaxf(s[0][0], s[1][0]);
+#pragma unroll
+    for (int i = 1; i < 16; ++i) mx = fmaxf(fmaxf(mx, s[0][i]), s[1][i]);
+    mx = half_max(mx);
+    // the exponent reference follows the running maximum only when it is
+    // passed by more than 2^kRefSlack (always on a row's first key)
+    const bool move = mx > kNegInf && !((mx - m_ref) * sc <= kRefSlack);
+    if (__ballot(move)) {
+      const float mn = move ? mx : m_ref;
+      const float alpha = !move ? 1.f : m_ref == kNegInf ? 0.f : __builtin_amdgcn_exp2f((m_ref - mn) * sc);
+      l_run *= alpha;
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) acc[dt][i] *= alpha;
+      m_ref = mn;
+    }
+    const float nb = m_ref == kNegInf ? 0.f : -m_ref * sc;
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      float sum = 0.f;
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        s[t][i] = __builtin_amdgcn_exp2f(fmaf(s[t][i], sc, nb));
+        sum += s[t][i];
+      }
+      l_run += sum;
+    }
+    // O^T += V^T P^T, 16 keys per step: element j of lane half h is key
+    // 8 (j / 4) + 4 h + j % 4 of the step in both operands
+#pragma unroll
+    for (int st = 0; st < kKeys / 16; ++st) {
+      u32x4 pw;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) pw[e] = pack_bf16x2(s[st >> 1][(st & 1) * 8 + 2 * e], s[st >> 1][(st & 1) * 8 + 2 * e + 1]);
+      const bf16x8 pB = as_bf16x8(pw);
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt) {
+        // 16-lane group (h, g): rows 4 h + 0..3 of the step (then + 8), dims 32 dt + 16 g .. + 15
+        const int i = lane & 15, g = (lane >> 4) & 1;
+        const int r = st * 16 + h * 4 + (i >> 2);
+        const int X = dt * 4 + g * 2 + ((i & 3) >> 1);
+        const unsigned char* src = vt + r * ROWB + ((X ^ vswz(r)) << 4) + (i & 1) * 8;
+        const uint2 lo = lds_read_tr(src);
+        const uint2 hi = lds_read_tr(src + 8 * ROWB);  // (vswz(r + 8) == vswz(r))
+        const bf16x8 vA = as_bf16x8(u32x4{lo.x, lo.y, hi.x, hi.y});
+        acc[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vA, pB, acc[dt], 0, 0, 0);
+      }
+    }
+  };
+
+  if (key_end > key_begin) {  // (uniform; a paged part past the table's last key has none)
+    issue(key_begin);
+    stage(0, key_begin);
+    lds_barrier();
+    int buf = 0;
+    for (int n0 = key_begin; n0 < key_end; n0 += kKeys, buf ^= 1) {
+      const bool more = n0 + kKeys < key_end;
+      if (more) issue(n0 + kKeys);
+      compute(buf, n0);
+      if (more) stage(buf ^ 1, n0 + kKeys);
+      lds_barrier();
+    }
+  }
+
+  // lane (h, col), element i of tile dt: O[row col][32 dt + 8 (i / 4) + 4 h + i % 4]
+  const float L = half_sum(l_run);
+  const float inv = L > 0.f ? 1.f / L : 0.f;
+  const int r = r0 + col;
+  if (slot >= 0) {  // one of several key ranges of the tile: an unnormalised partial for the merge
+    if (r >= nrows) return;
+    float* base = a.part + ((int64_t)slot * a.H + head) * a.tile_rows * (DH + 2);
+    float* dst = base + r * DH + h * 4;
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        *reinterpret_cast<f32x4*>(dst + dt * 32 + q * 8) =
+            f32x4{acc[dt][4 * q], acc[dt][4 * q + 1], acc[dt][4 * q + 2], acc[dt][4 * q + 3]};
+    if (h == 0) *reinterpret_cast<float2*>(base + a.tile_rows * DH + 2 * r) = make_float2(m_ref * sc, L);
+    return;
+  }
+  if (r < nrows) {
+    bf16_t* dst = a.out + ((int64_t)(row0 + r) * a.H + head) * DH + h * 4;
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const uint32_t lo = pack_bf16x2(acc[dt][4 * q] * inv, acc[dt][4 * q + 1] * inv);
+        const uint32_t hi = pack_bf16x2(acc[dt][4 * q + 2] * inv, acc[dt][4 * q + 3] * inv);
+        *reinterpret_cast<uint2*>(dst + dt * 32 + q * 8) = make_uint2(lo, hi);
+      }
+  }
+}
+
+// Merge of the tiles cut over keys: one workgroup per (tile, head, 256 /
+// (DH / 4) rows), one thread per (row, 4 dims):
+//   out = sum_s 2^(m_s - M) o_s / sum_s 2^(m_s - M) l_s, in part order.
+struct PrefillMergeArgs {
+  bf16_t* out;
+  const float* part;
+  const int32_t* merges;  // [nmerge][4]: first slot, parts, first row, rows
+  int H, tile_rows;
+};
+
+template <int DH>
+__global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillMergeArgs a) {
+  constexpr int C4 = DH / 4;
+  const int32_t* rec = a.merges + (int64_t)blockIdx.x * 4;
+  const int slot = rec[0], parts = rec[1], row0 = rec[2], nrows = rec[3];
+  const int head = blockIdx.y;
+  const int r = blockIdx.z * (256 / C4) + threadIdx.x / C4, c4 = threadIdx.x % C4;
+  if (r >= nrows) return;
+  const int64_t stride = (int64_t)a.H * a.tile_rows * (DH + 2);
+  const float* base = a.part + (int64_t)slot * stride + (int64_t)head * a.tile_rows * (DH + 2);
+  constexpr int CH = 4;  // parts per round trip
+  float M = kNegInf, den = 0.f;
+  f32x4 num = {0.f, 0.f, 0.f, 0.f};
+  for (int s0 = 0; s0 < parts; s0 += CH) {
+    float2 ml[CH];
+    f32x4 o[CH];
+#pragma unroll
+    for (int k = 0; k < CH; ++k) {
+      const float* p = base + min(s0 + k, parts - 1) * stride;
+      ml[k] = *reinterpret_cast<const float2*>(p + a.tile_rows * DH + 2 * r);
+      o[k] = *reinterpret_cast<const f32x4*>(p + r * DH + c4 * 4);
+    }
+    float Mn = M;
+#pragma unroll
+    for (int k = 0; k < CH; ++k) Mn = fmaxf(Mn, ml[k].x);  // (a part read twice changes nothing here)
+    if (Mn == kNegInf) continue;  // no key of this row so far
+    const float w0 = __builtin_amdgcn_exp2f(M - Mn);  // from -inf: 0
+    den *= w0;
+    num *= w0;
+#pragma unroll
+    for (int k = 0; k < CH; ++k) {
+      const float wk = s0 + k < parts ? __builtin_amdgcn_exp2f(ml[k].x - Mn) : 0.f;
+      den = fmaf(ml[k].y, wk, den);
+      num += o[k] * wk;
+    }
+    M = Mn;
+  }
+  const float inv = den > 0.f ? 1.f / den : 0.f;
+  bf16_t* dst = a.out + ((int64_t)(row0 + r) * a.H + head) * DH + c4 * 4;
+  *reinterpret_cast<uint2*>(dst) =
+      make_uint2(pack_bf16x2(num[0] * inv, num[1] * inv), pack_bf16x2(num[2] * inv, num[3] * inv));
+}
+
+}  // namespace
+
+extern "C" {
+
+int nsv_prefill_attention(void* out, const void* q, const void* k, const void* v, const int32_t* block_tables,
+                          const int32_t* tiles, int ntiles, int tile_rows, const int32_t* merges, int nmerges,
+                          float scale, int H, int Hkv, int D, int block_size, int max_blocks, void* partials,
+                          void* stream) {
+  if (ntiles < 0 || nmerges < 0 || H <= 0 || Hkv <= 0) return NSV_ERR_ARG;
+  if (H % Hkv || (D != 64 && D != 128)) return NSV_ERR_UNSUPPORTED;
+  const int G = H / Hkv, hw = G % 2 == 0 ? 2 : 1;
+  const int nw = tile_rows * hw / kWaveRows;
+  if ((nw != 8 && nw != 4) || nw * kWaveRows != tile_rows * hw) return NSV_ERR_UNSUPPORTED;
+  int bs_log2 = 0;
+  if (block_tables) {
+    if (max_blocks <= 0 || block_size <= 0 || (block_size & (block_size - 1))) return NSV_ERR_UNSUPPORTED;
+    while ((1 << bs_log2) < block_size) ++bs_log2;
+    if ((int64_t)max_blocks * block_size > ((int64_t)1 << 30)) return NSV_ERR_UNSUPPORTED;
+  }
+  if (ntiles == 0) return NSV_OK;
+  if (!out || !q || !k || !v || !tiles || (nmerges > 0 && !merges)) return NSV_ERR_ARG;
+  if (nmerges > 0 && !partials) return NSV_ERR_WORKSPACE;
+  const int64_t grid = (int64_t)ntiles * H / hw;
+  if (grid > 0x7fffffff) return NSV_ERR_UNSUPPORTED;
+  PrefillArgs a;
+  a.q = (const bf16_t*)q;
+  a.k = (const bf16_t*)k;
+  a.v = (const bf16_t*)v;
+  a.out = (bf16_t*)out;
+  a.block_tables = block_tables;
+  a.tiles = tiles;
+  a.scale_log2 = scale * 1.44269504088896340736f;
+  a.H = H;
+  a.Hkv = Hkv;
+  a.bs_log2 = bs_log2;
+  a.max_blocks = max_blocks;
+  a.hw = hw;
+  a.hgroups = G / hw;
+  a.part = (float*)partials;
+  a.tile_rows = tile_rows;
+  hipStream_t s = (hipStream_t)stream;
+  const dim3 g((unsigned)grid), b(nw * 64);
+  if (D == 128) {
+    if (nw == 8) hipLaunchKernelGGL((prefill_attn_kernel<128, 8>), g, b, 0, s, a);
+    else hipLaunchKernelGGL((prefill_attn_kernel<128, 4>), g, b, 0, s, a);
+  } else {
+    if (nw == 8) hipLaunchKernelGGL((prefill_attn_kernel<64, 8>), g, b, 0, s, a);
+    else hipLaunchKernelGGL((prefill_attn_kernel<64, 4>), g, b, 0, s, a);
+  }
+  const int rc = nsv_launch_status();
+  if (rc || nmerges == 0) return rc;
+  PrefillMergeArgs m;
+  m.out = (bf16_t*)out;
+  m.part = (const float*)partials;
+  m.merges = merges;
+  m.H = H;
+  m.tile_rows = tile_rows;
+  if (D == 128) hipLaunchKernelGGL(prefill_merge_kernel<128>, dim3(nmerges, H, tile_rows / 8), dim3(256), 0, s, m);
+  else hipLaunchKernelGGL(prefill_merge_kernel<64>, dim3(nmerges, H, tile_rows / 16), dim3(256), 0, s, m);
+  return nsv_launch_status();
+}
+
+}  // extern "C"

@@ -183,11 +183,143 @@ def store_kvcache(
     _lib.check(rc, "store_kvcache")
 
 
+_PREFILL_KEYS = 64    # keys per tile of the prefill kernel
+_PREFILL_PAGES = 2048  # block-table entries it stages for one record
+
+
+def prefill_tiles(seqlens_q, seqlens_k, num_heads: int, num_kv_heads: int, block_size: int | None, cus: int):
+    """The prefill kernel's work list (nsv_prefill_attention) for sequences of
+    seqlens_q new rows ending seqlens_k keys each; block_size None: K/V are
+    the sequences' keys back to back.  Host arithmetic only.
+    Returns (tiles [n, 8] int32, merges [m, 4] int32, tile_rows, slots).
+
+    Rows per tile: a workgroup of 8 waves of 32 rows (two query heads of a kv
+    head where the group is even) reads a K/V tile for twice the rows of a
+    4-wave one, but fewer, larger workgroups fill the chip worse and idle
+    longer at the causal edge.  Measured on MI355X, 4 against 8 waves: 8
+    prompts of ~1000 tokens (16/8 heads) 59 against 73 us, one of 1206 39
+    against 45, 4096 (32/8 heads) 180 against 161, two of 2900-4050 behind
+    4096 cached keys 870 against 781: 8 waves from 24 key tiles per record on
+    average.
+
+    Cut over keys: where the tiles alone are fewer than the compute units, a
+    record's chain of key tiles (~1.8 us each with one wave per SIMD) is the
+    call's time, so tiles longer than 1.5 targets are cut into parts of about
+    `target` key tiles and merged by a second kernel: 40 rows behind 4096
+    keys 114 -> 20 us (targets 3 and 4; 6: 21, 8: 24), 270 rows of 32/8 heads
+    120 -> 50-62 (16, 12), one prompt of 1206 40 -> 31 (4; 3: 35, 8: 34).
+    With more tiles than compute units the partials cost what the shorter
+    chain saves (1206 of 32/8 heads, 304 workgroups: 41.7 -> 39-43; 8 prompts
+    59 -> 64-172), so those stay whole."""
+    import numpy as np
+
+    ql, kl = np.asarray(seqlens_q, dtype=np.int64), np.asarray(seqlens_k, dtype=np.int64)
+    if len(ql) != len(kl):
+        raise ValueError("seqlens_q and seqlens_k differ in length")
+    bad = np.nonzero((ql <= 0) | (ql > kl))[0]
+    if len(bad):
+        raise ValueError(f"prefill sequence {bad[0]}: {ql[bad[0]]} query rows over {kl[bad[0]]} keys")
+    group = num_heads // num_kv_heads
+    hw = 2 if group % 2 == 0 else 1
+    q0, k0 = np.cumsum(ql) - ql, np.cumsum(kl) - kl
+
+    def cut(rows):
+        n = -(-ql // rows)  # tiles per sequence
+        seq = np.repeat(np.arange(len(ql)), n)
+        first = (np.arange(len(seq)) - np.repeat(np.cumsum(n) - n, n)) * rows  # first new row of the tile
+        nr = np.minimum(rows, ql[seq] - first)
+        pos = kl[seq] - ql[seq] + first
+        return seq, q0[seq] + first, nr, pos, -(-(pos + nr) // _PREFILL_KEYS)
+
+    rows = 8 * 32 // hw
+    seq, row0, nr, pos, nt = cut(rows)
+    if nt.sum() < 24 * len(nt):
+        rows //= 2
+        seq, row0, nr, pos, nt = cut(rows)
+    units = len(seq) * (num_heads // hw)
+    parts = np.ones_like(nt)
+    if units <= cus:
+        target = max(4, -(-int(nt.sum()) * (num_heads // hw) * 2 // (3 * cus)))
+        parts = np.where(2 * nt > 3 * target, -(-nt // target), parts)
+    if block_size is not None:  # a record's pages fit the kernel's LDS copy
+        parts = np.maximum(parts, -(-nt // max(1, (_PREFILL_PAGES - 1) * block_size // _PREFILL_KEYS)))
+    per = -(-nt // parts)
+    parts = -(-nt // per)
+    slot0 = np.cumsum(np.where(parts > 1, parts, 0)) - np.where(parts > 1, parts, 0)
+    cuts = parts > 1
+    merges = np.stack([slot0[cuts], parts[cuts], row0[cuts], nr[cuts]], axis=1).astype(np.int32)
+    t = np.repeat(np.arange(len(seq)), parts)  # the tile of each record
+    i = np.arange(len(t)) - np.repeat(np.cumsum(parts) - parts, parts)
+    begin = i * per[t] * _PREFILL_KEYS
+    end = np.minimum(pos[t] + nr[t], begin + per[t] * _PREFILL_KEYS)
+    kv0 = k0[seq[t]] if block_size is None else np.zeros_like(t)
+    tiles = np.stack([seq[t], row0[t], nr[t], pos[t], kv0, begin, end, np.where(cuts[t], slot0[t] + i, -1)], axis=1)
+    order = np.argsort(begin - end, kind="stable")  # heaviest first
+    return tiles[order].astype(np.int32), merges, rows, int(parts[cuts].sum())
+
+
+class PrefillPlan:
+    """The work list of one prefill step on the device, in one transfer."""
+
+    def __init__(self, seqlens_q, seqlens_k, num_heads: int, num_kv_heads: int, block_size: int | None, device):
+        import numpy as np
+
+        cus = torch.cuda.get_device_properties(device).multi_processor_count
+        tiles, merges, self.tile_rows, self.slots = prefill_tiles(seqlens_q, seqlens_k, num_heads, num_kv_heads,
+                                                                  block_size, cus)
+        self.num_heads, self.num_kv_heads, self.block_size = num_heads, num_kv_heads, block_size
+        self.sequences, self.rows, self.keys = len(seqlens_q), int(sum(seqlens_q)), int(sum(seqlens_k))
+        self.ntiles, self.nmerges = len(tiles), len(merges)
+        self.work = torch.from_numpy(np.concatenate([tiles.ravel(), merges.ravel()])).to(device)
+
+
+def prefill_attention(query: torch.Tensor, k: torch.Tensor, v: torch.Tensor, plan: PrefillPlan, scale: float,
+                      head_dim: int, block_tables: torch.Tensor | None = None) -> torch.Tensor:
+    """Causal attention of a prefill step's rows (bf16): query [rows, H, D];
+    k, v the step's own [keys, Hkv, D], or with block_tables the paged caches
+    [num_blocks, block_size, Hkv, D] (layers/attention.py:123-363)."""
+    H, Hkv = plan.num_heads, plan.num_kv_heads
+    if not query.is_cuda:
+        raise ValueError("prefill_attention runs on the GPU; query is on the CPU")
+    if query.dtype != torch.bfloat16 or k.dtype != query.dtype or v.dtype != query.dtype:
+        raise ValueError("query, k and v must be bfloat16")
+    if query.dim() != 3 or tuple(query.shape[1:]) != (H, head_dim) or query.shape[0] < plan.rows:
+        raise ValueError(f"query must be (at least {plan.rows}, {H}, {head_dim}), got {tuple(query.shape)}")
+    max_blocks = 0
+    if block_tables is None:
+        if tuple(k.shape) != tuple(v.shape) or tuple(k.shape[1:]) != (Hkv, head_dim) or k.shape[0] < plan.keys:
+            raise ValueError(f"k and v must be (at least {plan.keys}, {Hkv}, {head_dim}), got {tuple(k.shape)}")
+        k, v = k.contiguous(), v.contiguous()
+    else:
+        nb, bs, hkv, d = _check_cache(k, "k_cache")
+        if tuple(v.shape) != (nb, bs, hkv, d) or not v.is_contiguous():
+            raise ValueError("k_cache and v_cache must have the same contiguous shape")
+        if (bs, hkv, d) != (plan.block_size, Hkv, head_dim):
+            raise ValueError("cache shape disagrees with block_size / num_kv_heads / head_dim")
+        block_tables = _as(block_tables, "block_tables")
+        if block_tables.shape[0] < plan.sequences:
+            raise ValueError(f"{plan.sequences} sequences but {block_tables.shape[0]} block-table rows")
+        max_blocks = block_tables.shape[1]
+    query = query.contiguous()
+    out = torch.empty_like(query)
+    # (from the caching allocator on the current stream: calls on several
+    # streams or threads share nothing)
+    part = torch.empty(plan.slots * H * plan.tile_rows * (head_dim + 2), dtype=torch.float32,
+                       device=query.device) if plan.slots else None
+    tiles = plan.work.data_ptr()
+    rc = _lib.lib().nsv_prefill_attention(
+        out.data_ptr(), query.data_ptr(), k.data_ptr(), v.data_ptr(), _lib.ptr(block_tables), tiles, plan.ntiles,
+        plan.tile_rows, tiles + plan.ntiles * 32, plan.nmerges, float(scale), H, Hkv, head_dim,
+        plan.block_size or 1, max_blocks, _lib.ptr(part), _lib.stream_ptr(query.device))
+    _lib.check(rc, "prefill_attention")
+    return out
+
+
 _prefill_plan: tuple = (None, None)  # (the Context it was built for, its tensors)
 
 
 def _prefill_rows(ctx, num_heads: int, num_kv_heads: int, device) -> tuple:
-    """Verify-kernel metadata of a prefill step, built once per Context.
+    """Verify-kernel metadata of an fp32 prefill step, built once per Context.
 
     Sequence i has seqlens_q[i] new rows at positions seqlens_k[i] -
     seqlens_q[i] .. seqlens_k[i] - 1.  Its rows are cut into causal blocks of
@@ -244,8 +376,9 @@ class Attention(nn.Module):
         prompt behind a cached prefix) the keys come from the paged cache,
         the step's own K/V already stored in it, as the reference's
         paged_attention_prefill (:328-363); without, from the step's
-        contiguous K/V, as its varlen flash path (:257-325).  Both run on the
-        verify kernel over causal blocks of rows (``_prefill_rows``);
+        contiguous K/V, as its varlen flash path (:257-325).  bf16 runs on
+        the prefill kernel (``prefill_attention``), fp32 on the verify kernel
+        over causal blocks of rows (``_prefill_rows``);
       * decode (neither flag): one query row per sequence attending its
         whole context (:759-767), served by the same verify kernel with
         each row at position context_lens - 1."""
@@ -260,6 +393,25 @@ class Attention(nn.Module):
         self.block_size = block_size
         self.k_cache = self.v_cache = torch.tensor([])
 
+    def _prefill_bf16(self, context, q, k, v, scale: float) -> torch.Tensor:
+        """The prefill branch on the prefill kernel; the step's work list is
+        built by its first layer and kept with the step's Context."""
+        paged = context.block_tables is not None
+        if context.seqlens_q is None or context.seqlens_k is None:
+            raise ValueError("a prefill step needs context.seqlens_q and context.seqlens_k")
+        bs = self.block_size if paged else None
+        key = (self.num_heads, self.num_kv_heads, bs, q.device)
+        plans = context.__dict__.setdefault("prefill_plans", {})
+        plan = plans.get(key)
+        if plan is None:
+            plan = plans[key] = PrefillPlan(context.seqlens_q, context.seqlens_k, self.num_heads, self.num_kv_heads,
+                                            bs, q.device)
+        if paged:
+            return prefill_attention(q, self.k_cache, self.v_cache, plan, scale, self.head_dim,
+                                     context.block_tables.to(q.device))
+        return prefill_attention(q, k.reshape(-1, self.num_kv_heads, self.head_dim),
+                                 v.reshape(-1, self.num_kv_heads, self.head_dim), plan, scale, self.head_dim)
+
     def forward(self, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor) -> torch.Tensor:
         context = get_context()
         k_cache, v_cache = self.k_cache, self.v_cache
@@ -272,6 +424,9 @@ class Attention(nn.Module):
         if context.is_prefill and not context.is_verify:
             if context.cu_seqlens_q is None:
                 raise ValueError("cu_seqlens_q must be provided for varlen attention")
+            if q.dtype == torch.bfloat16:
+                o = self._prefill_bf16(context, q, k, v, scale)
+                return o.reshape(o.shape[0], self.num_heads * self.head_dim)
             bt, lens, cu, positions, q_block = _prefill_rows(context, self.num_heads, self.num_kv_heads, q.device)
             if context.block_tables is not None:
                 kc, vc, bs = k_cache, v_cache, self.block_size

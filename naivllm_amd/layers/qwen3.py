@@ -34,7 +34,7 @@ import torch
 import torch.nn.functional as F
 
 from naivllm_amd import _lib
-from naivllm_amd.layers.attention import paged_attention_verify
+from naivllm_amd.layers.attention import PrefillPlan, paged_attention_verify, prefill_attention
 
 
 @dataclass
@@ -308,12 +308,30 @@ class Qwen3Verify:
 
     @torch.inference_mode()
     def prefill(self, token_lists, starts, tables) -> torch.Tensor:
-        """One forward over the new tokens of several sequences (see
-        prefill_metadata): their K/V land in the paged cache, and the logits
-        of each sequence's last token come back, [len(token_lists), vocab]."""
-        ids, pos, slots, bt, ctx, cu, last = prefill_metadata(token_lists, starts, tables, self.block_size,
-                                                              self.prefill_q_block(), self.device)
-        return self.forward(ids, pos, slots, bt, ctx, cu, self.prefill_q_block(), logits_rows=last)
+        """One forward over the new tokens of several sequences (sequence i's
+        from starts[i] on; the pages before hold their K/V: a cached prefix):
+        their K/V land in the paged cache, and the logits of each sequence's
+        last token come back, [len(token_lists), vocab]."""
+        import numpy as np
+
+        bs, lens = self.block_size, [len(t) for t in token_lists]
+        for n, start in zip(lens, starts):
+            if not 0 <= start < n:
+                raise ValueError(f"prefill start {start} outside a {n}-token sequence")
+        new = [n - start for n, start in zip(lens, starts)]
+        pos = [np.arange(start, n, dtype=np.int64) for n, start in zip(lens, starts)]
+        slots = [np.asarray(t, dtype=np.int64)[p // bs] * bs + p % bs for t, p in zip(tables, pos)]
+        ids = [np.asarray(t[start:], dtype=np.int64) for t, start in zip(token_lists, starts)]
+        bt = np.full((len(tables), max(len(t) for t in tables)), -1, dtype=np.int32)
+        for row, t in zip(bt, tables):
+            row[:len(t)] = t
+        last = np.cumsum(new, dtype=np.int64) - 1
+        to = lambda x: torch.from_numpy(x).to(self.device)  # noqa: E731
+        rows = to(np.concatenate([*ids, *pos, *slots, last]))  # one transfer
+        T = sum(new)
+        plan = PrefillPlan(new, lens, self.cfg.num_heads, self.cfg.num_kv_heads, bs, self.device)
+        return self.forward(rows[:T], rows[T:2 * T], rows[2 * T:3 * T], to(bt), None, None, 0,
+                            logits_rows=rows[3 * T:], prefill=plan)
 
     def allocate_kv_cache(self, num_blocks: int, block_size: int) -> None:
         """One [num_blocks, block_size, Hkv, D] K and V pool per layer
@@ -327,25 +345,31 @@ class Qwen3Verify:
     def forward(self, input_ids: torch.Tensor, positions: torch.Tensor, slot_mapping: torch.Tensor,
                 block_tables: torch.Tensor, context_lens: torch.Tensor, cu_seqlens_q: torch.Tensor,
                 max_q_len: int, logits_out: torch.Tensor | None = None,
-                logits_rows: torch.Tensor | None = None) -> torch.Tensor:
+                logits_rows: torch.Tensor | None = None, prefill: PrefillPlan | None = None) -> torch.Tensor:
         """Verify forward over T = sum of per-sequence query rows.  Rows at
         position -1 are inert padding (no KV store, zero attention output).
         Returns logits [T, vocab] (written into logits_out when given), or
-        only the rows ``logits_rows`` indexes (the prefill's last rows)."""
+        only the rows ``logits_rows`` indexes (the prefill's last rows).
+        prefill: the rows are whole prompts' (block_tables then one row per
+        prompt; context_lens, cu_seqlens_q and max_q_len are not used)."""
         if self.dtype != torch.bfloat16:
             raise ValueError("the fused forward kernels are bf16")
         cfg = self.cfg
         H, Hkv, D, E = cfg.num_heads, cfg.num_kv_heads, cfg.head_dim, cfg.hidden_size
         eps = cfg.rms_norm_eps
         T = input_ids.shape[0]
-        block_m = max(16, 1 << (max_q_len - 1).bit_length())
         I = cfg.intermediate_size
         resid = torch.empty(T, E, dtype=self.dtype, device=self.device)  # the residual stream
         h = torch.empty_like(resid)
         q = torch.empty(T, H, D, dtype=self.dtype, device=self.device)
-        attn = lambda li: paged_attention_verify(  # noqa: E731
-            q, self.k_caches[li], self.v_caches[li], block_tables, context_lens, cu_seqlens_q, positions,
-            self.scale, H, Hkv, D, self.block_size, block_m, max_q_len=max_q_len)
+        if prefill is not None:
+            attn = lambda li: prefill_attention(  # noqa: E731
+                q, self.k_caches[li], self.v_caches[li], prefill, self.scale, D, block_tables)
+        else:
+            block_m = max(16, 1 << (max_q_len - 1).bit_length())
+            attn = lambda li: paged_attention_verify(  # noqa: E731
+                q, self.k_caches[li], self.v_caches[li], block_tables, context_lens, cu_seqlens_q, positions,
+                self.scale, H, Hkv, D, self.block_size, block_m, max_q_len=max_q_len)
         # embedding lookup, layer 0's input norm, and the rotary rows of the step's
         # positions (gathered once for every layer, so that each layer's epilogue
         # loads them without first loading the positions) in one launch
