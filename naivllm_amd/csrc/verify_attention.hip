@@ -27,7 +27,7 @@
 //     through its own L1 (shared in L2); the key splits of a slice, when
 //     used, merge in-kernel like the key-split kernel's (the last of them to
 //     finish), or in a second kernel past the arrival counters' capacity.
-// The fp32 kernel (the 1e-5 contract) uses VALU dot products.
+// The fp32 kernel (the 1e-5 contract) uses the fp32 matrix instruction.
 
 #include "common.h"
 
@@ -48,6 +48,8 @@ constexpr int kMaxSplitPages = 1024;  // block-table entries of one split staged
 // workspace.  The area has one fixed size, so every call finds its counters
 // at the same place, zero, whatever the previous call's shape was.
 constexpr int kMaxCounterPairs = 16384;
+// scratch of the allocation-free entry point
+constexpr size_t kNoAllocScratchBytes = (size_t)16 << 20;
 // Counter slot of a pair: pairs 0..255 each get their own 256-byte line
 // (device-scope atomics on one line serialise, ~20 ns apiece), and pair
 // p + 256 k shares p's line.
@@ -104,7 +106,6 @@ struct VerifyArgs {
   int Gs, g0;        // query heads per kv head, and the first of the G this launch serves
   int dqc;           // head-dim slices per pair (d-sliced bf16 kernel)
   int ks_splits;     // key-split kernel: splits per sequence when split_tokens == 0
-  int m_base;        // fp32 kernel: first query row (of the Mv) this launch serves
   int dmerge;        // d-sliced kernel: the pair's last workgroup merges its splits in-kernel (else a merge launch)
 #if NSV_STAMP
   unsigned long long* stamps;  // [grid][kStampSlots] of this launch, or null
@@ -1547,21 +1548,52 @@ __global__ __launch_bounds__(NW * 64, 8 / NW) void verify_attn_ks_kernel(VerifyA
   }
 }
 
-// fp32 path: one wave per workgroup, VALU dot products (exact fp32 math, the
-// 1e-5 contract).  Lane = key for Q.K, lane = head dim for P.V.
+// fp32 path (the 1e-5 contract): fp32 products and sums throughout, on the
+// fp32 matrix instruction (v_mfma_f32_16x16x4_f32).
+//
+// A short call is bound by its chain of memory round trips, a long one by
+// HBM (16 rows of 16 keys take 2,048 matrix cycles per 16 KiB of K/V).  A
+// workgroup serves one (pair, key split) with four waves that take 16-key
+// tiles in turn.  Every operand is loaded as 16-byte pieces straight into
+// the matrix layout, because a contraction may number its terms in any order
+// as long as both operands agree:
+//   S^T = K Q^T   lane (g, c): K[key c][16 j + 4 g + e] is term 4 j + e's
+//                 slot g, and so is Q (staged once per workgroup in LDS);
+//   O^T = V^T P^T step i takes keys 4 g + i: P is this lane's own score i,
+//                 and V[key 4 g + i][64 h + 4 c + e] feeds output tile
+//                 (h, e), whose row c is dim 64 h + 4 c + e.
+// So nothing is transposed or shuffled, and K/V never pass through LDS.
+// One wave per workgroup with a key per lane before (8 pairs x 1,248 keys,
+// 18 rows): 344 us per graph-replayed call, merge included; now 14.1 with 20
+// splits (17.0 with 10, 24.1 with 5).  8 sequences 36.8 us (7 splits; 39.5
+// with 10, 44.6 with 3); 16 sequences x 4,096 keys 186 us at 48 rows and 101
+// (5.3 TB/s) at 4 rows per pair.
 // ---------------------------------------------------------------------------
+constexpr int kF32Waves = 4;
+
 template <int MT, int DH>
-__global__ __launch_bounds__(64) void verify_attn_f32_kernel(VerifyArgs a) {
+__global__ __launch_bounds__(kF32Waves * 64, 2) void verify_attn_f32_kernel(VerifyArgs a) {
+  constexpr int NW = kF32Waves, NT = NW * 64;
   constexpr int MP = MT * 16;
-  constexpr int E = DH / 64;
-  __shared__ __attribute__((aligned(16))) float q_s[MP][DH];
-  __shared__ float p_s[MP][NSV_WAVE];
-  __shared__ int pos_s[MP];
+  constexpr int KJ = DH / 16;              // 16-byte K pieces per lane and tile
+  constexpr int VH = DH / 64;              // 16-byte V pieces per lane and key
+  constexpr int NS = MT <= 2 ? 2 : 1;      // tiles in flight (registers)
+  constexpr int QSTR = DH + 4;             // staged row strides (floats): a 16-byte read of 16 rows
+  constexpr int RSTR = DH + 4;             // falls in distinct banks
+  constexpr int QF = MP * QSTR, RF = NW * 16 * RSTR;
+  struct __attribute__((aligned(16))) Lds {
+    float buf[QF > RF ? QF : RF];          // the query rows, then one row tile of every wave's O
+    float red_m[NW][MP], red_l[NW][MP];
+    float row_m[MP], row_l[MP];
+  };
+  __shared__ Lds lds;
 
   int split, pair;
   decode_block(a, split, pair);
   if (pair >= a.npairs) return;
-  const int lane = threadIdx.x;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int g = lane >> 4, c = lane & 15;
   const int b = pair / a.Hkv, hk = pair - b * a.Hkv;
   const int ctx = context_len(a, b);
   const int nsplit = num_splits(a, ctx);
@@ -1571,29 +1603,22 @@ __global__ __launch_bounds__(64) void verify_attn_f32_kernel(VerifyArgs a) {
   const int q0 = uniform(a.cu_seqlens_q[b]);
   const int qlen = uniform(a.cu_seqlens_q[b + 1]) - q0;
 
-  // local row r serves query row m = m_base + r of the pair's Mv rows
-  for (int idx = lane; idx < MP * DH; idx += NSV_WAVE) {
-    const int r = idx / DH, d = idx - r * DH;
-    const int m = a.m_base + r;
-    const int g = m / a.QL, t = m - g * a.QL;
-    const bool ok = (m < a.Mv) && (t < qlen);
-    q_s[r][d] = ok ? ((const float*)a.q)[((int64_t)(q0 + t) * a.H + hk * a.Gs + a.g0 + g) * DH + d] : 0.f;
+  // query row m = g * QL + t of the group; rows past the group or the sequence are zero
+  for (int idx = tid; idx < MP * (DH / 4); idx += NT) {
+    const int m = idx / (DH / 4), ch = idx % (DH / 4);
+    const int gh = m / a.QL, t = m - gh * a.QL;
+    f32x4 v = {0.f, 0.f, 0.f, 0.f};
+    if (m < a.Mv && t < qlen)
+      v = *reinterpret_cast<const f32x4*>((const float*)a.q +
+                                          ((int64_t)(q0 + t) * a.H + hk * a.Gs + a.g0 + gh) * DH + ch * 4);
+    *reinterpret_cast<f32x4*>(&lds.buf[m * QSTR + ch * 4]) = v;
   }
-  if (lane < MP) {
-    const int m = a.m_base + lane;
-    const int g = m / a.QL, t = m - g * a.QL;
-    const bool ok = (m < a.Mv) && (t < qlen);
-    pos_s[lane] = ok ? load_pos(a.positions, q0 + t) : -1;
-  }
-  __syncthreads();
-
-  float m_run[MP], l_run[MP], acc[MP][E];
+  int pos[MT];  // position of this lane's row c of each row tile
 #pragma unroll
-  for (int m = 0; m < MP; ++m) {
-    m_run[m] = kNegInf;
-    l_run[m] = 0.f;
-#pragma unroll
-    for (int e = 0; e < E; ++e) acc[m][e] = 0.f;
+  for (int mt = 0; mt < MT; ++mt) {
+    const int m = mt * 16 + c;
+    const int gh = m / a.QL, t = m - gh * a.QL;
+    pos[mt] = m < a.Mv && t < qlen ? load_pos(a.positions, q0 + t) : -1;
   }
 
   const int32_t* bt = a.block_tables + (int64_t)b * a.max_blocks;
@@ -1602,85 +1627,162 @@ __global__ __launch_bounds__(64) void verify_attn_f32_kernel(VerifyArgs a) {
   const float* kbase = (const float*)a.k_cache + hk * DH;
   const float* vbase = (const float*)a.v_cache + hk * DH;
 
-  for (int n0 = tok_begin; n0 < tok_end; n0 += NSV_WAVE) {
-    const int n = n0 + lane;
-    int blk = -1;
-    if (n < tok_end) blk = bt[n >> a.bs_log2];
-    const bool ok = blk >= 0;
-    float s[MP];
+  struct Tile {
+    f32x4 k[KJ];      // K[key c][16 j + 4 g ..]
+    f32x4 v[4][VH];   // V[key 4 g + i][64 h + 4 c ..]
+    unsigned mask;    // keys of the tile that exist (inside the split, page mapped)
+  };
+  auto issue = [&](Tile& T, int n0) {
+    const int n = n0 + c;
+    int pg = -1;
+    if (n < tok_end) pg = bt[n >> a.bs_log2];
+    T.mask = (unsigned)__ballot(pg >= 0) & 0xffffu;
+    // a key that does not exist reads the tile's first one that does (its weight is zero); none: nothing is read
+    if (T.mask == 0) return;  // uniform
+    const int first = __builtin_ctz(T.mask);
+    const int pg_first = __shfl(pg, first, NSV_WAVE);
+    auto row = [&](int key, int page) {  // element offset of a key's row
+      const int64_t p = page >= 0 ? page : pg_first;
+      const int nn = n0 + (page >= 0 ? key : first);
+      return ((p << a.bs_log2) + (nn & bs_mask)) * tok_stride;
+    };
+    const float* kp = kbase + row(c, pg) + 4 * g;
 #pragma unroll
-    for (int m = 0; m < MP; ++m) s[m] = 0.f;
-    if (ok) {
-      const float* kp = kbase + ((int64_t)blk * (bs_mask + 1) + (n & bs_mask)) * tok_stride;
-      for (int d = 0; d < DH; d += 4) {
-        const float4 kv = *reinterpret_cast<const float4*>(kp + d);
+    for (int j = 0; j < KJ; ++j) T.k[j] = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(kp + 16 * j));
 #pragma unroll
-        for (int m = 0; m < MP; ++m) {
-          const float4 qv = *reinterpret_cast<const float4*>(&q_s[m][d]);
-          s[m] = fmaf(qv.x, kv.x, s[m]);
-          s[m] = fmaf(qv.y, kv.y, s[m]);
-          s[m] = fmaf(qv.z, kv.z, s[m]);
-          s[m] = fmaf(qv.w, kv.w, s[m]);
-        }
+    for (int i = 0; i < 4; ++i) {
+      const float* vp = vbase + row(4 * g + i, __shfl(pg, 4 * g + i, NSV_WAVE)) + 4 * c;
+#pragma unroll
+      for (int h = 0; h < VH; ++h) T.v[i][h] = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(vp + 64 * h));
+    }
+  };
+
+  float m_run[MT], l_run[MT];
+  f32x4 acc[MT][VH][4];  // [h][e]: element i is O[row c][64 h + 16 g + 4 i + e]
+#pragma unroll
+  for (int mt = 0; mt < MT; ++mt) {
+    m_run[mt] = kNegInf;
+    l_run[mt] = 0.f;
+#pragma unroll
+    for (int h = 0; h < VH; ++h)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) acc[mt][h][e] = f32x4{0.f, 0.f, 0.f, 0.f};
+  }
+  auto compute = [&](const Tile& T, int n0) {
+    if (T.mask == 0) return;  // uniform
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) {
+      f32x4 s = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int j = 0; j < KJ; ++j) {
+        const f32x4 qv = *reinterpret_cast<const f32x4*>(&lds.buf[(mt * 16 + c) * QSTR + 16 * j + 4 * g]);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) s = __builtin_amdgcn_mfma_f32_16x16x4f32(T.k[j][e], qv[e], s, 0, 0, 0);
       }
-    }
+      // element i: key 4 g + i, row c
+      float mx = kNegInf;
 #pragma unroll
-    for (int m = 0; m < MP; ++m) {
-      const float x = (ok && n <= pos_s[m]) ? s[m] * a.scale_log2 : kNegInf;
-      const float m_new = fmaxf(m_run[m], wave_max(x));
-      const float ms = (m_new == kNegInf) ? 0.f : m_new;
-      const float alpha = exp2f(m_run[m] - ms);
-      const float p = exp2f(x - ms);
-      l_run[m] = l_run[m] * alpha + wave_sum(p);
-      m_run[m] = m_new;
-#pragma unroll
-      for (int e = 0; e < E; ++e) acc[m][e] *= alpha;
-      p_s[m][lane] = p;
-    }
-    __syncthreads();
-    const int jn = min(NSV_WAVE, tok_end - n0);
-    for (int j = 0; j < jn; ++j) {
-      const int nn = n0 + j;
-      const int bj = bt[nn >> a.bs_log2];
-      if (bj < 0) continue;  // uniform across the wave
-      const float* vp = vbase + ((int64_t)bj * (bs_mask + 1) + (nn & bs_mask)) * tok_stride;
-      float v[E];
-#pragma unroll
-      for (int e = 0; e < E; ++e) v[e] = vp[lane + 64 * e];
-#pragma unroll
-      for (int m = 0; m < MP; ++m) {
-        const float p = p_s[m][j];
-#pragma unroll
-        for (int e = 0; e < E; ++e) acc[m][e] = fmaf(p, v[e], acc[m][e]);
+      for (int i = 0; i < 4; ++i) {
+        const int key = 4 * g + i;
+        s[i] = ((T.mask >> key) & 1) && n0 + key <= pos[mt] ? s[i] * a.scale_log2 : kNegInf;
+        mx = fmaxf(mx, s[i]);
       }
+      const float m_new = fmaxf(m_run[mt], row_max4(mx));
+      const float ms = m_new == kNegInf ? 0.f : m_new;
+      const float alpha = exp2f(m_run[mt] - ms);
+      float sum = 0.f;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        s[i] = exp2f(s[i] - ms);
+        sum += s[i];
+      }
+      l_run[mt] = l_run[mt] * alpha + row_sum4(sum);
+      m_run[mt] = m_new;
+      if (__ballot(alpha != 1.f)) {
+#pragma unroll
+        for (int h = 0; h < VH; ++h)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) acc[mt][h][e] *= alpha;
+      }
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int h = 0; h < VH; ++h)
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            acc[mt][h][e] = __builtin_amdgcn_mfma_f32_16x16x4f32(T.v[i][h][e], s[i], acc[mt][h][e], 0, 0, 0);
     }
-    __syncthreads();
+  };
+
+  constexpr int STEP = 16 * NW;  // keys the workgroup's waves take per turn
+  Tile T[NS];
+  issue(T[0], tok_begin + w * 16);
+  __syncthreads();  // query rows staged
+  for (int n0 = tok_begin + w * 16; n0 < tok_end; n0 += NS * STEP) {
+    if constexpr (NS == 2) {
+      issue(T[1], n0 + STEP);  // (past the split: an empty tile)
+      compute(T[0], n0);
+      issue(T[0], n0 + 2 * STEP);
+      compute(T[1], n0 + STEP);
+    } else {
+      compute(T[0], n0);
+      issue(T[0], n0 + STEP);
+    }
   }
 
-  if (nsplit == 1) {
-    float* out = (float*)a.out;
+  // ---- the waves' rows combined, one row tile at a time through LDS
+  if (g == 0) {
 #pragma unroll
-    for (int r = 0; r < MP; ++r) {
-      const int m = a.m_base + r;
-      const int g = m / a.QL, t = m - g * a.QL;
-      if (m >= a.Mv || t >= qlen) continue;
-#pragma unroll
-      for (int e = 0; e < E; ++e)
-        out[((int64_t)(q0 + t) * a.H + hk * a.Gs + a.g0 + g) * DH + lane + 64 * e] =
-            l_run[r] > 0.f ? acc[r][e] / l_run[r] : 0.f;
+    for (int mt = 0; mt < MT; ++mt) {
+      lds.red_m[w][mt * 16 + c] = m_run[mt];
+      lds.red_l[w][mt * 16 + c] = l_run[mt];
     }
-    return;
   }
-  const int64_t base = ((int64_t)pair * a.S + split) * a.Mv + a.m_base;
+  __syncthreads();  // (also: every wave is done with the staged query rows)
+  if (tid < MP) {
+    float M = kNegInf, L = 0.f;
 #pragma unroll
-  for (int r = 0; r < MP; ++r) {
-    if (a.m_base + r >= a.Mv) continue;
+    for (int ww = 0; ww < NW; ++ww) M = fmaxf(M, lds.red_m[ww][tid]);
+    const float ref = M == kNegInf ? 0.f : M;
 #pragma unroll
-    for (int e = 0; e < E; ++e) a.part_o[(base + r) * DH + lane + 64 * e] = acc[r][e];
-    if (lane == 0) {
-      a.part_ml[(base + r) * 2 + 0] = m_run[r];
-      a.part_ml[(base + r) * 2 + 1] = l_run[r];
+    for (int ww = 0; ww < NW; ++ww) L += lds.red_l[ww][tid] * exp2f(lds.red_m[ww][tid] - ref);
+    lds.row_m[tid] = M;
+    lds.row_l[tid] = L;
+  }
+  __syncthreads();
+  const int64_t base = ((int64_t)pair * a.S + split) * a.Mv;
+#pragma unroll
+  for (int mt = 0; mt < MT; ++mt) {
+    const float M = lds.row_m[mt * 16 + c];
+    const float f = M == kNegInf ? 0.f : exp2f(m_run[mt] - M);
+    float* dst = &lds.buf[(w * 16 + c) * RSTR + 16 * g];
+#pragma unroll
+    for (int h = 0; h < VH; ++h)
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        *reinterpret_cast<f32x4*>(dst + 64 * h + 4 * i) =
+            f32x4{acc[mt][h][0][i], acc[mt][h][1][i], acc[mt][h][2][i], acc[mt][h][3][i]} * f;
+    __syncthreads();
+    for (int idx = tid; idx < 16 * (DH / 4); idx += NT) {
+      const int r = idx / (DH / 4), ch = idx % (DH / 4), m = mt * 16 + r;
+      const int gh = m / a.QL, t = m - gh * a.QL;
+      if (m >= a.Mv) continue;
+      f32x4 o = *reinterpret_cast<const f32x4*>(&lds.buf[r * RSTR + ch * 4]);
+#pragma unroll
+      for (int ww = 1; ww < NW; ++ww) o += *reinterpret_cast<const f32x4*>(&lds.buf[(ww * 16 + r) * RSTR + ch * 4]);
+      if (nsplit > 1) {
+        *reinterpret_cast<f32x4*>(&a.part_o[(base + m) * DH + ch * 4]) = o;
+      } else if (t < qlen) {
+        const float L = lds.row_l[m];
+        *reinterpret_cast<f32x4*>((float*)a.out + ((int64_t)(q0 + t) * a.H + hk * a.Gs + a.g0 + gh) * DH + ch * 4) =
+            L > 0.f ? o / L : f32x4{0.f, 0.f, 0.f, 0.f};
+      }
     }
+    __syncthreads();
+  }
+  if (nsplit > 1 && tid < a.Mv) {
+    a.part_ml[(base + tid) * 2 + 0] = lds.row_m[tid];
+    a.part_ml[(base + tid) * 2 + 1] = lds.row_l[tid];
   }
 }
 
@@ -1921,9 +2023,18 @@ int make_plan(int B, int H, int Hkv, int D, int block_size, int max_blocks, int 
       return NSV_ERR_UNSUPPORTED;
     }
   } else if (split == 0) {
-    // fp32: enough one-wave workgroups to cover the chip a few times over
+    // fp32: splits of 256 keys, doubled while the pairs alone give the chip
+    // a few workgroups per CU ...
     split = 256;
     while (pairs * ((max_ctx + split - 1) / split) > 1024 && split < 8192) split *= 2;
+    // ... and cut down to 64 (one 16-key tile per wave) while the grid is
+    // under two workgroups per CU (8 pairs x 1,248 keys: 64-key splits 14.1
+    // us, 128 17.0, 256 24.1; 64 pairs: 192 36.8, 256 40.4), as long as the partials stay within what
+    // the allocation-free entry point holds (no shape it took is refused)
+    const int64_t fine = std::max<int64_t>(64, (max_ctx * pairs / (2 * (int64_t)cus) + 63) / 64 * 64);
+    const int64_t fine_s = (max_ctx + fine - 1) / fine;
+    if (fine < split && (int64_t)kMaxCounterPairs * 4 + pairs * fine_s * p->Mv * (D + 2) * 4 + 256 <= kNoAllocScratchBytes)
+      split = fine;
   }
   p->split = (int)split;
   p->S = (int)((max_ctx + split - 1) / split);
@@ -1986,25 +2097,12 @@ int launch_bf16(const VerifyArgs& a, int D, dim3 grid, hipStream_t s) {
   return NSV_ERR_UNSUPPORTED;
 }
 
-// fp32: at most two 16-row tiles per launch; more query rows per pair run
-// as further launches over the next 32 rows (the single-launch form for 64
-// rows, 256 VGPRs + 254 AGPRs of row state per lane, returned wrong rows on
-// MI355X; two launches read the pair's K/V twice, which the 1e-5 path can
-// afford).
 template <int MT>
 void launch_f32(const VerifyArgs& a, int D, dim3 grid, hipStream_t s) {
-  if constexpr (MT <= 2) {
-    if (D == 128)
-      hipLaunchKernelGGL((verify_attn_f32_kernel<MT, 128>), grid, dim3(64), 0, s, a);
-    else
-      hipLaunchKernelGGL((verify_attn_f32_kernel<MT, 64>), grid, dim3(64), 0, s, a);
-  } else {
-    VerifyArgs b = a;
-    b.m_base = 0;
-    launch_f32<2>(b, D, grid, s);
-    b.m_base = 32;
-    launch_f32<MT - 2>(b, D, grid, s);
-  }
+  if (D == 128)
+    hipLaunchKernelGGL((verify_attn_f32_kernel<MT, 128>), grid, dim3(kF32Waves * 64), 0, s, a);
+  else
+    hipLaunchKernelGGL((verify_attn_f32_kernel<MT, 64>), grid, dim3(kF32Waves * 64), 0, s, a);
 }
 
 // ---------------------------------------------------------------------------
@@ -2084,7 +2182,6 @@ __global__ __launch_bounds__(512) void stream_read_kernel(const char* buf, size_
 // library runs on gets its own copy, at its own address, for the life of
 // the process.  Device globals start zeroed and every call leaves the
 // counters zero, the invariant the workspace contract already relies on.
-constexpr size_t kNoAllocScratchBytes = (size_t)16 << 20;
 static __device__ __attribute__((aligned(256))) unsigned char scratch[kNoAllocScratchBytes];
 
 constexpr int kMaxScratchDevices = 64;
@@ -2266,7 +2363,6 @@ int nsv_verify_attention(void* out, const void* q, const void* k_cache, const vo
   a.P8 = (B * Hkv + 7) / 8;
   a.dqc = p.dqc;
   a.ks_splits = p.ks_splits;
-  a.m_base = 0;
   // the d-sliced kernel merges its key splits in-kernel while every pair has
   // an arrival counter of its own, else in a second launch
   a.dmerge = dtype == NSV_BF16 && !p.ks && p.S > 1 && (int64_t)B * Hkv * p.dqc <= kMaxCounterPairs;

@@ -241,3 +241,18 @@ def test_repeated_calls_share_the_workspace(split):
         g.replay()
         torch.cuda.synchronize()
         assert_close(out, want, "bf16", f"graph split {split}")
+
+
+@pytest.mark.parametrize("G,ql,D,bs", [(1, 1, 128, 1), (2, 9, 128, 16), (4, 9, 64, 4), (4, 12, 128, 256), (4, 16, 64, 64),
+                                       (4, 16, 128, 16)])
+def test_fp32_tile_edges(G, ql, D, bs):
+    # one to four row tiles of the fp32 kernel, contexts around a 16-key tile,
+    # a 64-key split and a turn of its four waves, an unmapped page
+    print(f"case: fp32 {G} heads x {ql} rows, D={D} page={bs}", flush=True)
+    ctx = [max(ql, n) for n in (1, 15, 16, 17, 63, 64, 65, 129, 321)]
+    vb = synth.verify_batch(41, ctx, [min(ql, n) for n in ctx], num_heads=2 * G, num_kv_heads=2, head_dim=D,
+                            block_size=bs, dtype="f32")
+    if bs <= 64:
+        vb.block_tables[8, 2] = -1
+    out = _gpu(vb, max_q_len=ql)
+    assert_close(out, _oracle(vb), "f32", "fp32 edges")
