@@ -86,3 +86,26 @@ def test_drop_in_draft_appends_to_sequences():
     assert seqs[0].draft_tokens == [8, 9, 1] and seqs[0].token_ids == prompt + [8, 9, 1]
     assert seqs[0].num_tokens == len(prompt) + 3 and seqs[0].last_token == 1
     assert seqs[1].draft_tokens == [] and seqs[1].num_tokens == 2
+
+
+@pytest.mark.parametrize("L", [2, 3, 1023, 1024, 1025, 1026, 2049, 12289, 36863, 36864, 36865, 40000])
+def test_history_lengths_around_the_blocks(L):
+    # the scan's blocks of 1024 tokens and the staged history's capacity: rare
+    # tokens with a planted quote, a repeated token, and hits inside tokens
+    print(f"case: ngram history of {L}", flush=True)
+    rare = [int(x) for x in synth.randint(L, 72, L, 0, 1 << 30)]
+    at = L // 3
+    n = min(5, L - 1 - at)
+    if n > 0:
+        rare[L - n:] = rare[at:at + n]
+    few = np.array([0x01010101, 0x01010100, 0x00010101, 1, 256], dtype=np.int64)
+    bytes_ = [int(few[x]) for x in synth.randint(L + 1, 73, L, 0, 5)]
+    # one hit inside a token, the aligned match it hides, and another below it
+    hidden = list(rare)
+    if L > 1000:
+        hidden[-2:] = [0x22222222, 0x22222222]
+        hidden[L // 2:L // 2 + 4] = [0x11222222, 0x22222222, 0x22222222, 0x33333333]
+        hidden[10:12] = [0x22222222, 0x22222222]
+    hs = [rare, [7] * L, bytes_, hidden]
+    for (k, lo, hi) in [(8, 2, 8), (4, 1, 3)]:
+        assert run(hs, k, lo, hi, stride=L + 3) == on.draft(hs, k, lo, hi)
