@@ -459,6 +459,37 @@ int nsv_linear_decode(const void* x, const void* norm_w, const float* ss_in,
                       int epilogue, void* stream);
 int nsv_linear_decode_ss_rows(int M, int N);
 
+/* Projections of up to 128 rows whose weights one pass streams (the verify
+ * rows of several sequences at wide hidden sizes, the LM head past the rows
+ * nsv_lm_head takes); references as nsv_linear's, without its fusions.
+ *   epilogue 0: y [M, N] = x W^T (bf16, fp32 accumulation); where
+ *     nsv_wide_linear_splits is s > 1 the reduction is cut over s workgroups
+ *     and partials [s, M, N] fp32 is written instead of y, to be summed in
+ *     split order and rounded once by nsv_rms_norm_sum or
+ *     nsv_qk_norm_rope_store_sum.
+ *   epilogue 1 (SiluAndMul): W holds [gate; up] ([N = 2I, K]); y [M, I] =
+ *     silu(gate) * up, gate and up rounded to bf16 first.
+ *   packed != 0: W in nsv_lm_head_pack's layout (epilogue 0; K of 1024, 2048
+ *     or 4096; one split).
+ * N % 16 == 0 (32 with epilogue 1), K % 256 == 0, M <= 128.
+ * nsv_wide_linear_splits (host only) is 0 for a shape that is not taken. */
+int nsv_wide_linear_splits(int M, int N, int K, int epilogue, int packed);
+int nsv_wide_linear(const void* x, const void* weight, void* y,
+                    float* partials, int M, int N, int K, int epilogue,
+                    int packed, void* stream);
+/* nsv_rms_norm and nsv_qk_norm_rope_store (per-row rotary table) over the sum
+ * of a split projection's partials: x (or qkv) = bf16(sum of partials
+ * [splits, T, E] in split order).  E % 4 == 0, E <= 4096; residual given. */
+int nsv_rms_norm_sum(const float* partials, int splits, const void* residual,
+                     void* residual_out, const void* weight, void* out, int T,
+                     int E, float eps, void* stream);
+int nsv_qk_norm_rope_store_sum(const float* partials, int splits,
+                               const void* q_norm_w, const void* k_norm_w,
+                               const float* cos_sin,
+                               const int64_t* slot_mapping, void* q_out,
+                               void* k_cache, void* v_cache, int T, int H,
+                               int Hkv, int D, float eps, void* stream);
+
 /* The LM head (reference: src/myvllm/layers/embedding_head.py:71-83,
  * ParallelLMHead.forward's F.linear(x, weight) over the vocabulary rows) on
  * a weight repacked once at load time.  nsv_lm_head_pack writes the [N, K]

@@ -74,6 +74,10 @@ SIGNATURES: dict[str, tuple] = {
     "nsv_linear_decode": (_c_int, [_c_vp, _c_vp, _c_vp, _c_int, _c_f32, _c_vp, _c_vp, _c_vp, _c_vp]
                           + [_c_int] * 4 + [_c_vp]),
     "nsv_linear_decode_ss_rows": (_c_int, [_c_int] * 2),
+    "nsv_wide_linear_splits": (_c_int, [_c_int] * 5),
+    "nsv_wide_linear": (_c_int, [_c_vp] * 4 + [_c_int] * 5 + [_c_vp]),
+    "nsv_rms_norm_sum": (_c_int, [_c_vp, _c_int] + [_c_vp] * 4 + [_c_int] * 2 + [_c_f32, _c_vp]),
+    "nsv_qk_norm_rope_store_sum": (_c_int, [_c_vp, _c_int] + [_c_vp] * 7 + [_c_int] * 4 + [_c_f32, _c_vp]),
     "nsv_lm_head_rows": (_c_int, [_c_int] * 2),
     "nsv_lm_head_pack": (_c_int, [_c_vp, _c_vp, _c_int, _c_int, _c_vp]),
     "nsv_lm_head": (_c_int, [_c_vp, _c_vp, _c_vp, _c_int, _c_int, _c_int, _c_vp]),

@@ -72,6 +72,79 @@ __global__ __launch_bounds__(kNormThreads) void rms_norm_residual_kernel(
 }
 
 // ---------------------------------------------------------------------------
+// The same from a projection's fp32 partial sums (nsv_wide_linear with a
+// split reduction): x = bf16(sum over the splits, in split order), one
+// rounding as the unsplit projection's.  One workgroup per row, 16-byte
+// loads, 4 splits in flight per round trip: the splits cost no launch.
+// ---------------------------------------------------------------------------
+template <int J>  // 4-element groups per thread: E <= 1024 J
+__global__ __launch_bounds__(kNormThreads) void rms_norm_sum_kernel(
+    const float* __restrict__ part, int splits, const uint16_t* __restrict__ residual,
+    uint16_t* __restrict__ residual_out, const uint16_t* __restrict__ w, uint16_t* __restrict__ out, int T, int E,
+    float eps) {
+  __shared__ float red[kNormThreads / 64];
+  const int64_t row = blockIdx.x;
+  const int64_t stride = (int64_t)T * E;
+  int at[J];
+  uint2 rv[J], wv[J];
+  f32x4 v[J];
+#pragma unroll
+  for (int j = 0; j < J; ++j) {
+    at[j] = min(((int)threadIdx.x + j * kNormThreads) * 4, E - 4);
+    rv[j] = *reinterpret_cast<const uint2*>(residual + row * E + at[j]);
+    wv[j] = *reinterpret_cast<const uint2*>(w + at[j]);
+    v[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  }
+  for (int s0 = 0; s0 < splits; s0 += 4) {
+    f32x4 p[4][J];
+#pragma unroll
+    for (int s = 0; s < 4; ++s)
+#pragma unroll
+      for (int j = 0; j < J; ++j)
+        p[s][j] = *reinterpret_cast<const f32x4*>(part + min(s0 + s, splits - 1) * stride + row * E + at[j]);
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+      if (s0 + s >= splits) break;  // uniform
+#pragma unroll
+      for (int j = 0; j < J; ++j) v[j] += p[s][j];
+    }
+  }
+  float ss = 0.f;
+#pragma unroll
+  for (int j = 0; j < J; ++j) {
+    const bool in = ((int)threadIdx.x + j * kNormThreads) * 4 < E;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const uint32_t word = (e < 2 ? rv[j].x : rv[j].y) >> (16 * (e & 1)) & 0xffffu;
+      const float x = bf16_bits_to_f32(f32_to_bf16_bits(v[j][e]));
+      v[j][e] = bf16_bits_to_f32(f32_to_bf16_bits(x + bf16_bits_to_f32(word)));  // the residual stream is bf16
+      ss += in ? v[j][e] * v[j][e] : 0.f;
+    }
+  }
+  ss = wave_sum(ss);
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = ss;
+  __syncthreads();
+  float tot = 0.f;
+#pragma unroll
+  for (int i = 0; i < kNormThreads / 64; ++i) tot += red[i];
+  const float inv = rsqrtf(tot / (float)E + eps);
+#pragma unroll
+  for (int j = 0; j < J; ++j) {
+    if (((int)threadIdx.x + j * kNormThreads) * 4 >= E) continue;
+    float o[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const uint32_t word = (e < 2 ? wv[j].x : wv[j].y) >> (16 * (e & 1)) & 0xffffu;
+      o[e] = v[j][e] * inv * bf16_bits_to_f32(word);
+    }
+    if (residual_out)
+      *reinterpret_cast<uint2*>(residual_out + row * E + at[j]) =
+          make_uint2(pack_bf16x2(v[j][0], v[j][1]), pack_bf16x2(v[j][2], v[j][3]));
+    *reinterpret_cast<uint2*>(out + row * E + at[j]) = make_uint2(pack_bf16x2(o[0], o[1]), pack_bf16x2(o[2], o[3]));
+  }
+}
+
+// ---------------------------------------------------------------------------
 // Forward prologue: r = embed[ids[t]] (the residual stream's first value,
 // written to residual_out), out = rmsnorm(r) * w (layer 0's input norm), and
 // the rotary table row of the row's position (position < 0 takes row 0) into
@@ -139,6 +212,8 @@ __global__ __launch_bounds__(kNormThreads) void embed_norm_kernel(
 // ---------------------------------------------------------------------------
 struct EpilogueArgs {
   const uint16_t* qkv;
+  const float* part;     // [splits, T, heads * D]: the projection's partial sums instead of qkv (SUM)
+  int splits;
   const uint16_t* q_w;
   const uint16_t* k_w;
   const float* cos_sin;  // [max_pos, D]: cos in [0, D/2), sin in [D/2, D); [T, D] by row without positions
@@ -157,7 +232,9 @@ struct EpilogueArgs {
 // position.  Loads are unconditional (lanes past D/2 and waves past the last
 // head read clamped elements and leave): a load under a branch is waited for
 // on the spot.
-template <bool POS>
+// SUM: the row comes as a split projection's fp32 partial sums, added in
+// split order and rounded once, as the unsplit projection's output.
+template <bool POS, bool SUM = false>
 __global__ __launch_bounds__(256) void qk_norm_rope_store_kernel(EpilogueArgs a) {
   __asm__ volatile("" ::"s"(a.qkv), "s"(a.q_w), "s"(a.k_w), "s"(a.cos_sin), "s"(a.positions), "s"(a.slots),
                    "s"(a.q_out), "s"(a.k_cache), "s"(a.v_cache), "s"(a.T), "s"(a.H), "s"(a.Hkv), "s"(a.D),
@@ -171,9 +248,23 @@ __global__ __launch_bounds__(256) void qk_norm_rope_store_kernel(EpilogueArgs a)
   const bool on = lane < half;
   const int l = on ? lane : half - 1;
   const bool is_q = head < a.H, is_v = head >= a.H + a.Hkv;
-  const uint16_t* src = a.qkv + ((int64_t)row * heads + head) * a.D;
+  const int64_t at = ((int64_t)row * heads + head) * a.D;
   const uint16_t* w = is_q ? a.q_w : a.k_w;
-  const uint16_t s1 = src[l], s2 = src[l + half];
+  uint16_t s1, s2;
+  constexpr int CH = 8;  // splits per round trip
+  float p1[CH], p2[CH];
+  const int64_t stride = (int64_t)a.T * heads * a.D;
+  if constexpr (SUM) {
+#pragma unroll
+    for (int s = 0; s < CH; ++s) {
+      const float* src = a.part + min(s, a.splits - 1) * stride + at;
+      p1[s] = src[l];
+      p2[s] = src[l + half];
+    }
+  } else {
+    s1 = a.qkv[at + l];
+    s2 = a.qkv[at + l + half];
+  }
   const int64_t slot = a.slots[row];
   const uint16_t w1 = w[l], w2 = w[l + half];
   int64_t pos = row;
@@ -182,6 +273,26 @@ __global__ __launch_bounds__(256) void qk_norm_rope_store_kernel(EpilogueArgs a)
     pos = pos < 0 ? 0 : (pos >= a.max_pos ? a.max_pos - 1 : pos);
   }
   const float c = a.cos_sin[pos * a.D + l], sn = a.cos_sin[pos * a.D + half + l];
+  if constexpr (SUM) {
+    float x1 = 0.f, x2 = 0.f;
+    for (int s0 = 0; s0 < a.splits; s0 += CH) {  // uniform
+      if (s0 > 0) {
+#pragma unroll
+        for (int s = 0; s < CH; ++s) {
+          const float* src = a.part + min(s0 + s, a.splits - 1) * stride + at;
+          p1[s] = src[l];
+          p2[s] = src[l + half];
+        }
+      }
+#pragma unroll
+      for (int s = 0; s < CH; ++s) {
+        x1 += s0 + s < a.splits ? p1[s] : 0.f;
+        x2 += s0 + s < a.splits ? p2[s] : 0.f;
+      }
+    }
+    s1 = f32_to_bf16_bits(x1);
+    s2 = f32_to_bf16_bits(x2);
+  }
   // (used here, so that no load is moved behind the branches below, which
   // only some heads take)
   __asm__ volatile("" ::"v"(s1), "v"(s2), "v"(w1), "v"(w2), "v"(c), "v"(sn));
@@ -273,7 +384,7 @@ int nsv_qk_norm_rope_store(const void* qkv, const void* q_norm_w, const void* k_
   if (!qkv || !q_norm_w || !k_norm_w || !cos_sin || !slot_mapping || !q_out || !k_cache || !v_cache)
     return NSV_ERR_ARG;
   if (!positions && max_pos < T) return NSV_ERR_ARG;  // the per-row table has a row per step row
-  EpilogueArgs a{(const uint16_t*)qkv, (const uint16_t*)q_norm_w, (const uint16_t*)k_norm_w, cos_sin, positions,
+  EpilogueArgs a{(const uint16_t*)qkv, nullptr, 0, (const uint16_t*)q_norm_w, (const uint16_t*)k_norm_w, cos_sin, positions,
                  slot_mapping, (uint16_t*)q_out, (uint16_t*)k_cache, (uint16_t*)v_cache, T, H, Hkv, D, max_pos, eps};
   const int64_t waves = (int64_t)T * (H + 2 * Hkv);
   if (positions)
@@ -282,6 +393,39 @@ int nsv_qk_norm_rope_store(const void* qkv, const void* q_norm_w, const void* k_
   else
     hipLaunchKernelGGL(qk_norm_rope_store_kernel<false>, dim3((unsigned)((waves + 3) / 4)), dim3(256), 0,
                        (hipStream_t)stream, a);
+  return nsv_launch_status();
+}
+
+int nsv_rms_norm_sum(const float* partials, int splits, const void* residual, void* residual_out, const void* weight,
+                     void* out, int T, int E, float eps, void* stream) {
+  if (T < 0 || E <= 0 || splits < 1) return NSV_ERR_ARG;
+  if (E % 4 || E > 16 * kNormThreads) return NSV_ERR_UNSUPPORTED;
+  if (T == 0) return NSV_OK;
+  if (!partials || !residual || !weight || !out) return NSV_ERR_ARG;
+  const int J = (E + 4 * kNormThreads - 1) / (4 * kNormThreads);
+#define NSV_NORM_SUM(JJ)                                                                                          \
+  hipLaunchKernelGGL(rms_norm_sum_kernel<JJ>, dim3(T), dim3(kNormThreads), 0, (hipStream_t)stream, partials,     \
+                     splits, (const uint16_t*)residual, (uint16_t*)residual_out, (const uint16_t*)weight,        \
+                     (uint16_t*)out, T, E, eps)
+  if (J <= 1) NSV_NORM_SUM(1);
+  else if (J <= 2) NSV_NORM_SUM(2);
+  else NSV_NORM_SUM(4);
+#undef NSV_NORM_SUM
+  return nsv_launch_status();
+}
+
+int nsv_qk_norm_rope_store_sum(const float* partials, int splits, const void* q_norm_w, const void* k_norm_w,
+                               const float* cos_sin, const int64_t* slot_mapping, void* q_out, void* k_cache,
+                               void* v_cache, int T, int H, int Hkv, int D, float eps, void* stream) {
+  if (T < 0 || H <= 0 || Hkv <= 0 || D <= 0 || (D & 1) || D > 128 || splits < 1) return NSV_ERR_ARG;
+  if (T == 0) return NSV_OK;
+  if (!partials || !q_norm_w || !k_norm_w || !cos_sin || !slot_mapping || !q_out || !k_cache || !v_cache)
+    return NSV_ERR_ARG;
+  EpilogueArgs a{nullptr, partials, splits, (const uint16_t*)q_norm_w, (const uint16_t*)k_norm_w, cos_sin, nullptr,
+                 slot_mapping, (uint16_t*)q_out, (uint16_t*)k_cache, (uint16_t*)v_cache, T, H, Hkv, D, T, eps};
+  const int64_t waves = (int64_t)T * (H + 2 * Hkv);
+  hipLaunchKernelGGL((qk_norm_rope_store_kernel<false, true>), dim3((unsigned)((waves + 3) / 4)), dim3(256), 0,
+                     (hipStream_t)stream, a);
   return nsv_launch_status();
 }
 

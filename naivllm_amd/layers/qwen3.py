@@ -11,12 +11,14 @@ layer: the QKV projection (with the input RMSNorm as its prologue), the
 pre-attention epilogue (q/k RMSNorm + RoPE + paged KV store), verify
 attention, o_proj (with the residual add as its epilogue), gate_up
 (post-attention RMSNorm prologue, SiLU * up epilogue) and down (residual
-add epilogue).  Wider batches run the projections on hipBLASLt between
-this library's residual-RMSNorm, epilogue, attention and SiLU kernels.  The
-LM head runs on this library's streaming kernel up to lm_head_rows() rows
-(79 at hidden 1024, 19 at hidden 4096: the activations staged in one CU's
-LDS), from a copy of its weight packed in that kernel's load order, and on
-hipBLASLt beyond.  Weights are random (seeded): no checkpoint is
+add epilogue).  Up to WIDE_ROWS rows they run on the weight-streaming
+projections (8 launches per layer), wider batches on hipBLASLt between this
+library's residual-RMSNorm, epilogue, attention and SiLU kernels.  The LM
+head runs on this library's streaming kernel up to lm_head_rows() rows (79 at
+hidden 1024, 19 at hidden 4096: the activations staged in one CU's LDS), from
+a copy of its weight packed in that kernel's load order, on the
+weight-streaming kernel from the same copy up to WIDE_ROWS, and on hipBLASLt
+beyond.  Weights are random (seeded): no checkpoint is
 loaded.
 
 The forward takes the verify metadata explicitly (positions, slots, block
@@ -172,6 +174,49 @@ def linear(x: torch.Tensor, weight: torch.Tensor, y: torch.Tensor | None = None,
     _lib.check(rc, "linear")
 
 
+def wide_splits(M: int, N: int, K: int, swiglu: bool = False, packed: bool = False) -> int:
+    """Workgroups nsv_wide_linear cuts the reduction over (0: not its shape)."""
+    return int(_lib.lib().nsv_wide_linear_splits(M, N, K, int(swiglu), int(packed)))
+
+
+def wide_linear(x: torch.Tensor, weight: torch.Tensor, y: torch.Tensor | None, partials: torch.Tensor | None = None, *,
+                swiglu: bool = False, packed: bool = False) -> None:
+    """y = x @ weight.T on the weight-streaming kernel of up to 128 rows
+    (nsv_wide_linear); with wide_splits > 1 the fp32 partial sums go to
+    ``partials`` ([splits, M, N] at its start) instead.  swiglu: weight is
+    [gate; up] and y = silu(gate) * up.  packed: weight in the LM head's
+    packed layout."""
+    M, K = x.shape
+    N = weight.shape[0]
+    if weight.shape[1] != K or not (x.is_contiguous() and weight.is_contiguous()):
+        raise ValueError(f"wide_linear: x [M, K] and weight [N, K], contiguous; got {tuple(x.shape)}, "
+                         f"{tuple(weight.shape)}")
+    rc = _lib.lib().nsv_wide_linear(x.data_ptr(), weight.data_ptr(), _lib.ptr(y), _lib.ptr(partials), M, N, K,
+                                    int(swiglu), int(packed), _lib.stream_ptr(x.device))
+    _lib.check(rc, "wide_linear")
+
+
+def rms_norm_sum(partials: torch.Tensor, splits: int, weight: torch.Tensor, eps: float, out: torch.Tensor,
+                 residual: torch.Tensor, residual_out: torch.Tensor | None = None) -> None:
+    """rms_norm whose x is the sum of a split projection's partials."""
+    T, E = out.shape
+    rc = _lib.lib().nsv_rms_norm_sum(partials.data_ptr(), splits, residual.data_ptr(), _lib.ptr(residual_out),
+                                     weight.data_ptr(), out.data_ptr(), T, E, eps, _lib.stream_ptr(out.device))
+    _lib.check(rc, "rms_norm_sum")
+
+
+def qk_norm_rope_store_sum(partials, splits: int, q_norm_w, k_norm_w, rope_rows, slot_mapping, q_out, k_cache, v_cache,
+                           H: int, Hkv: int, D: int, eps: float) -> None:
+    """qk_norm_rope_store (one rotary row per step row) whose qkv is the sum
+    of a split projection's partials."""
+    T = q_out.shape[0]
+    rc = _lib.lib().nsv_qk_norm_rope_store_sum(
+        partials.data_ptr(), splits, q_norm_w.data_ptr(), k_norm_w.data_ptr(), rope_rows.data_ptr(),
+        slot_mapping.data_ptr(), q_out.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), T, H, Hkv, D, eps,
+        _lib.stream_ptr(q_out.device))
+    _lib.check(rc, "qk_norm_rope_store_sum")
+
+
 def silu_mul(gate_up: torch.Tensor, out: torch.Tensor) -> None:
     rc = _lib.lib().nsv_silu_mul(gate_up.data_ptr(), out.data_ptr(), gate_up.shape[0], out.shape[1],
                                  _lib.stream_ptr(gate_up.device))
@@ -187,6 +232,16 @@ def silu_mul(gate_up: torch.Tensor, out: torch.Tensor) -> None:
 # 4096 the fused kernel wins at 9 rows and loses from about 16.
 FUSED_ROWS = 80
 FUSED_ROWS_WIDE = 12  # hidden size above 2048
+
+
+# Rows, past the fused kernel's, up to which the projections and the LM head
+# run on the weight-streaming kernel (nsv_wide_linear): beyond, the activations
+# each workgroup re-reads cost what the library GEMM's larger tiles save.
+# Measured on MI355X at hidden 4096, graph-replayed over rotating weights, the
+# library against it: 72 rows qkv 23.1 -> 17.0 us, o 16.2 -> 11.5, gate_up with
+# SiLU 53.5 + 4 -> 46, down 42.9 -> 25.5, LM head 283 -> 239; 108 rows 23.7 ->
+# 21.2, 16.4 -> 14.1, 55 + 4 -> 55, 43.1 -> 30.6, 291 -> 282.
+WIDE_ROWS = 128
 
 
 # Rows up to which the LM head runs on this library's kernels: nsv_linear
@@ -306,6 +361,17 @@ class Qwen3Verify:
         up to 64 (GQA group x rows) per (sequence, kv head)."""
         return 64 // (self.cfg.num_heads // self.cfg.num_kv_heads)
 
+    def _wide_splits(self, T: int) -> tuple[int, int, int] | None:
+        """Splits of the qkv, o and down projections where T rows run on the
+        weight-streaming kernel, else None."""
+        cfg = self.cfg
+        E, I, HD = cfg.hidden_size, cfg.intermediate_size, cfg.num_heads * cfg.head_dim
+        if T > WIDE_ROWS or E % 4 or E > 4096 or not all(
+                L[k].is_contiguous() for L in self.layers for k in ("qkv", "o", "gate_up", "down")):
+            return None
+        n = (wide_splits(T, HD + 2 * cfg.num_kv_heads * cfg.head_dim, E), wide_splits(T, E, HD), wide_splits(T, E, I))
+        return n if min(*n, wide_splits(T, 2 * I, E, swiglu=True)) > 0 else None
+
     @torch.inference_mode()
     def prefill(self, token_lists, starts, tables) -> torch.Tensor:
         """One forward over the new tokens of several sequences (sequence i's
@@ -399,6 +465,38 @@ class Qwen3Verify:
                 linear(resid, L["gate_up"], act, norm_w=L["ln2"], ss_in=ss_o, eps=eps, swiglu=True, decode=dec)
                 linear(act, L["down"], resid=resid, ss_out=ss_d, decode=dec)
             rms_norm(resid, self.norm, eps, h)
+        elif (splits := self._wide_splits(T)) is not None:
+            # a few sequences' rows at wide hidden sizes: the weight-streaming
+            # kernel, whose split reductions the next kernel sums (8 launches
+            # per layer)
+            s_qkv, s_o, s_d = splits
+            nq = (H + 2 * Hkv) * D
+            f32 = dict(dtype=torch.float32, device=self.device)
+            part = torch.empty(max((s * n for s, n in ((s_qkv, nq), (s_o, E), (s_d, E)) if s > 1), default=0) * T, **f32)
+            qkv = torch.empty(T, nq, dtype=self.dtype, device=self.device)
+            act = torch.empty(T, I, dtype=self.dtype, device=self.device)
+            x = torch.empty_like(resid)
+
+            def add_norm(splits, weight, residual_out):  # h = rmsnorm(resid + the projection's output)
+                if splits > 1:
+                    rms_norm_sum(part, splits, weight, eps, h, resid, residual_out)
+                else:
+                    rms_norm(x, weight, eps, h, residual=resid, residual_out=residual_out)
+
+            for li, L in enumerate(self.layers):
+                wide_linear(h, L["qkv"], qkv, part)
+                if s_qkv > 1:
+                    qk_norm_rope_store_sum(part, s_qkv, L["q_norm"], L["k_norm"], rope_rows, slot_mapping, q,
+                                           self.k_caches[li], self.v_caches[li], H, Hkv, D, eps)
+                else:
+                    qk_norm_rope_store(qkv, L["q_norm"], L["k_norm"], rope_rows, None, slot_mapping, q,
+                                       self.k_caches[li], self.v_caches[li], H, Hkv, D, eps)
+                wide_linear(attn(li).view(T, H * D), L["o"], x, part)
+                add_norm(s_o, L["ln2"], resid)
+                wide_linear(h, L["gate_up"], act, swiglu=True)
+                wide_linear(act, L["down"], x, part)
+                last = li + 1 == len(self.layers)
+                add_norm(s_d, self.norm if last else self.layers[li + 1]["ln1"], None if last else resid)
         else:
             # wider batches: hipBLASLt projections between this library's
             # norm / epilogue / SiLU kernels (9 launches per layer)
@@ -418,8 +516,8 @@ class Qwen3Verify:
             h = h.index_select(0, logits_rows)
             T = h.shape[0]
         # the LM head: this library's streaming kernel up to lm_head_rows rows
-        # (it streams the vocabulary's weight rows faster there), hipBLASLt's
-        # large tiles beyond
+        # (activations whole in LDS), the weight-streaming kernel on the same
+        # packed copy up to WIDE_ROWS, hipBLASLt's large tiles beyond
         if T <= lm_head_rows(E):
             if logits_out is None:
                 logits_out = torch.empty(T, self.lm_head.shape[0], dtype=self.dtype, device=self.device)
@@ -427,6 +525,11 @@ class Qwen3Verify:
                 lm_head(h, self.lm_head_packed, logits_out)
             else:
                 linear(h, self.lm_head, logits_out)
+            return logits_out
+        if self.lm_head_packed is not None and T <= WIDE_ROWS and wide_splits(T, *self.lm_head.shape, packed=True):
+            if logits_out is None:
+                logits_out = torch.empty(T, self.lm_head.shape[0], dtype=self.dtype, device=self.device)
+            wide_linear(h, self.lm_head_packed, logits_out, packed=True)
             return logits_out
         if logits_out is None:
             return F.linear(h, self.lm_head)
