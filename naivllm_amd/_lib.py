@@ -137,6 +137,20 @@ def ptr(t: torch.Tensor | None) -> int | None:
     return None if t is None else t.data_ptr()
 
 
+def upload(x, device: torch.device) -> torch.Tensor:
+    """A contiguous numpy array's values on the device, on the current stream
+    and without waiting for it: through pinned memory of torch's host
+    allocator, which reuses a block only when its copies are done.  (A
+    pageable copy makes the host wait for everything enqueued before it, so a
+    prefill step's launches could not run ahead of the device.)  Inside a
+    capture the copy stays a waited-for one, which the capture refuses: a
+    replay would read host memory that has been reused."""
+    t = torch.from_numpy(x)
+    if torch.device(device).type != "cuda" or torch.cuda.is_current_stream_capturing():
+        return t.to(device)
+    return t.pin_memory().to(device, non_blocking=True)
+
+
 _workspaces: dict = {}
 _retired: list = []
 

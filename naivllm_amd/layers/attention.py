@@ -270,7 +270,7 @@ class PrefillPlan:
         self.num_heads, self.num_kv_heads, self.block_size = num_heads, num_kv_heads, block_size
         self.sequences, self.rows, self.keys = len(seqlens_q), int(sum(seqlens_q)), int(sum(seqlens_k))
         self.ntiles, self.nmerges = len(tiles), len(merges)
-        self.work = torch.from_numpy(np.concatenate([tiles.ravel(), merges.ravel()])).to(device)
+        self.work = _lib.upload(np.concatenate([tiles.ravel(), merges.ravel()]), device)
 
 
 def prefill_attention(query: torch.Tensor, k: torch.Tensor, v: torch.Tensor, plan: PrefillPlan, scale: float,

@@ -392,11 +392,10 @@ class Qwen3Verify:
         for row, t in zip(bt, tables):
             row[:len(t)] = t
         last = np.cumsum(new, dtype=np.int64) - 1
-        to = lambda x: torch.from_numpy(x).to(self.device)  # noqa: E731
-        rows = to(np.concatenate([*ids, *pos, *slots, last]))  # one transfer
+        rows = _lib.upload(np.concatenate([*ids, *pos, *slots, last]), self.device)
         T = sum(new)
         plan = PrefillPlan(new, lens, self.cfg.num_heads, self.cfg.num_kv_heads, bs, self.device)
-        return self.forward(rows[:T], rows[T:2 * T], rows[2 * T:3 * T], to(bt), None, None, 0,
+        return self.forward(rows[:T], rows[T:2 * T], rows[2 * T:3 * T], _lib.upload(bt, self.device), None, None, 0,
                             logits_rows=rows[3 * T:], prefill=plan)
 
     def allocate_kv_cache(self, num_blocks: int, block_size: int) -> None:

@@ -98,3 +98,20 @@ def test_rejects_oversized_batches_and_drafts():
     s.draft_tokens = s.draft_tokens + [1]  # K + 1 drafts
     with pytest.raises(ValueError):
         runner.run_spec_verify([s])
+
+
+def test_calls_in_a_row_keep_their_own_inputs():
+    # more calls than host staging copies, none waited for: each call's rows
+    # reach its own replay
+    print("case: run_spec_verify back to back", flush=True)
+    model, seqs = setup(7)
+    runner = ModelRunner(model, max_num_sequences=4, num_spec_tokens=K, max_model_length=256)
+    calls = [[seqs[0]], seqs, [seqs[2], seqs[1]]] * 4
+    want = []
+    for c in calls[:3]:
+        want.append(runner.run_spec_verify(c).clone())
+        torch.cuda.synchronize()
+    got = [runner.run_spec_verify(c).clone() for c in calls]
+    torch.cuda.synchronize()
+    for i, g in enumerate(got):
+        assert torch.equal(g, want[i % 3]), i
