@@ -22,9 +22,12 @@
 // Measured on MI355X (the verify kernel on causal blocks of 64 / G rows,
 // which every prefill ran on before -> this kernel): 8 prompts of ~1000
 // tokens, 16/8 heads, 538 -> 59 us (557 TFLOP/s); prompts of 2900 and 4050
-// tokens behind 4096 cached keys, 32/8 heads, 5283 -> 781 us (858); 8192
-// tokens, 32/8 heads, 590 us (932); one prompt of 1206 tokens, 16/8 heads,
-// 85 -> 31 us.
+// tokens behind 4096 cached keys, 32/8 heads, 5283 -> 725 us (924); 8192
+// tokens, 32/8 heads, 535 us (1028); one prompt of 1206 tokens, 16/8 heads,
+// 85 -> 31 us.  With K/V staged through registers instead of straight to LDS
+// and both waves of a SIMD in step: 59-64, 781-793, 590 and 31 us (counters:
+// matrix cores and VALU 42% busy each, nearly one after the other; 34% of the
+// wave cycles waiting).
 
 #include "common.h"
 
@@ -83,14 +86,20 @@ __global__ __launch_bounds__(NW * 64, 2) void prefill_attn_kernel(PrefillArgs a)
   constexpr int ROWB = DH * 2;             // bytes per staged row
   constexpr int KS = DH / 16;              // k-steps of S^T
   constexpr int DT = DH / 32;              // 32-dim tiles of O^T
-  constexpr int LD = kKeys * CPR / NT;     // 16-byte K (and V) loads per thread and tile
+  constexpr int RPI = 64 / CPR;            // rows one load instruction of a wave fills
+  constexpr int J = kKeys / RPI / NW;      // K (and V) loads per wave and tile
   constexpr int TILEB = kKeys * ROWB;
-  static_assert(LD >= 1 && kKeys * CPR % NT == 0, "whole tiles per pass");
+  constexpr bool SKEW = NW == 8;           // see the loop
+  // tiles loading ahead, and the K and V tiles staged for it: two ahead with
+  // one workgroup per CU; one ahead for two 4-wave workgroups to fit a CU
+  constexpr int DIST = SKEW ? 2 : 1;
+  constexpr int KB = DIST + 1, VB = DIST + 1 + SKEW;
+  static_assert(J >= 1 && kKeys % (RPI * NW) == 0, "whole tiles per pass");
   struct __attribute__((aligned(16))) Lds {
     int pages[kMaxPages];
-    int holes;
-    __attribute__((aligned(16))) unsigned char kt[2][TILEB];
-    __attribute__((aligned(16))) unsigned char vt[2][TILEB];
+    int holes, first;  // some page unmapped; first mapped page
+    __attribute__((aligned(16))) unsigned char kt[KB][TILEB];
+    __attribute__((aligned(16))) unsigned char vt[VB][TILEB];
   };
   __shared__ Lds lds;
 
@@ -128,7 +137,10 @@ __global__ __launch_bounds__(NW * 64, 2) void prefill_attn_kernel(PrefillArgs a)
 
   const int pg0 = key_begin >> a.bs_log2;    // first page staged
   if (paged) {
-    if (tid == 0) lds.holes = 0;
+    if (tid == 0) {
+      lds.holes = 0;
+      lds.first = kMaxPages;
+    }
     __syncthreads();
     const int npg = ((key_end + bs_mask) >> a.bs_log2) - pg0;
     const int32_t* bt = a.block_tables + (int64_t)seq * a.max_blocks + pg0;
@@ -140,36 +152,51 @@ __global__ __launch_bounds__(NW * 64, 2) void prefill_attn_kernel(PrefillArgs a)
     __syncthreads();
   }
   const bool holes = paged && __builtin_amdgcn_readfirstlane(lds.holes) != 0;
+  int64_t spare = 0;  // the row an unmapped key reads instead (of a key that exists; its weight is zero)
+  if (holes) {        // uniform
+    const int npg = ((key_end + bs_mask) >> a.bs_log2) - pg0;
+    for (int i = tid; i < npg; i += NT)
+      if (lds.pages[i] >= 0) atomicMin(&lds.first, i);
+    __syncthreads();
+    const int first = __builtin_amdgcn_readfirstlane(lds.first);
+    if (first == kMaxPages) key_end = key_begin;  // no key at all
+    else spare = (int64_t)lds.pages[first] << a.bs_log2;
+  }
 
-  // K/V rows of a tile: thread -> rows tid / CPR + j NT / CPR, chunk tid % CPR
-  const int lr = tid / CPR, lc = tid % CPR;
-  u32x4 kr[LD], vr[LD];
-  auto issue = [&](int n0) {
+  // K/V rows of a tile go from memory straight to LDS (no registers, no LDS
+  // stores): instruction j of wave w fills rows (w J + j) RPI .. with 16-byte
+  // chunk X of row r at slot X ^ (r % CPR) (K), X ^ 4 (r % 4) (V), so that the
+  // operand reads of a half-wave touch every bank once; the lane picks the
+  // chunk its slot holds.  Rows past the last key read it again (masked).
+  auto vswz = [](int r) { return ((r & 3) << 2) & (CPR - 1); };
+  // (Issued from asm: the compiler would wait for every such load before the
+  // next LDS read of any buffer.  The loads have no register result; the
+  // waits below and the barriers order them.)
+  auto load_lds = [&](const bf16_t* src, unsigned char* dst) {
+    const uint32_t at = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)dst);
+    __asm__ volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(at), "v"(src) : "memory");
+  };
+  auto issue = [&](int kb, int vb, int n0) {
 #pragma unroll
-    for (int j = 0; j < LD; ++j) {
-      const int key = n0 + lr + j * (NT / CPR);
-      const int kc = min(key, key_end - 1);
+    for (int j = 0; j < J; ++j) {
+      const int r0j = (w * J + j) * RPI;
+      const int r = r0j + lane / CPR, sl = lane % CPR;
+      const int kc = min(n0 + r, key_end - 1);
       int64_t row = kv0 + kc;
-      if (paged) row = ((int64_t)max(lds.pages[(kc >> a.bs_log2) - pg0], 0) << a.bs_log2) + (kc & bs_mask);
-      const int64_t off = row * tok + hk * DH + lc * 8;
-      kr[j] = *reinterpret_cast<const u32x4*>(a.k + off);
-      vr[j] = *reinterpret_cast<const u32x4*>(a.v + off);
+      if (paged) {
+        const int p = lds.pages[(kc >> a.bs_log2) - pg0];
+        row = p >= 0 ? ((int64_t)p << a.bs_log2) + (kc & bs_mask) : spare;
+      }
+      const int64_t off = row * tok + hk * DH;
+      load_lds(a.k + off + ((sl ^ (r & (CPR - 1))) << 3), &lds.kt[kb][r0j * ROWB]);
+      load_lds(a.v + off + ((sl ^ vswz(r)) << 3), &lds.vt[vb][r0j * ROWB]);
     }
   };
-  // K chunk X of key r at slot X ^ (r % CPR); V chunk X at X ^ 4 (r % 4): the
-  // operand reads of a half-wave then touch every bank once
-  auto vswz = [](int r) { return ((r & 3) << 2) & (CPR - 1); };
-  auto stage = [&](int buf, int n0) {
-#pragma unroll
-    for (int j = 0; j < LD; ++j) {
-      const int r = lr + j * (NT / CPR);
-      const int key = n0 + r;
-      bool ok = key < key_end;
-      if (holes && ok) ok = lds.pages[(key >> a.bs_log2) - pg0] >= 0;
-      const u32x4 zero = {0u, 0u, 0u, 0u};
-      *reinterpret_cast<u32x4*>(&lds.kt[buf][r * ROWB + ((lc ^ (r & (CPR - 1))) << 4)]) = ok ? kr[j] : zero;
-      *reinterpret_cast<u32x4*>(&lds.vt[buf][r * ROWB + ((lc ^ vswz(r)) << 4)]) = ok ? vr[j] : zero;
-    }
+  // tile n0's loads landed, `ahead` tiles after it still in flight (the
+  // wave's own; the barrier that follows makes the tile whole)
+  auto landed = [&](bool ahead) {
+    if (DIST == 2 && ahead) __asm__ volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * J) : "memory");
+    else __asm__ volatile("s_waitcnt vmcnt(0)" ::: "memory");
   };
 
   f32x16 acc[DT];
@@ -180,34 +207,61 @@ __global__ __launch_bounds__(NW * 64, 2) void prefill_attn_kernel(PrefillArgs a)
   float m_ref = kNegInf, l_run = 0.f;
   const float sc = a.scale_log2;
 
-  auto compute = [&](int buf, int n0) {
-    if (n0 > pos_last) return;  // uniform: every key lies past this wave's rows
-    const unsigned char* kt = lds.kt[buf];
-    const unsigned char* vt = lds.vt[buf];
-    f32x16 s[2];
+  f32x16 s[2];
+  // scores of a tile (every key of a skipped tile lies past this wave's rows)
+  auto scores = [&](int kb, int n0) {
+    if (n0 > pos_last) return;  // uniform
+    const unsigned char* kt = lds.kt[kb];
+    // K operands KH steps at a time, both 32-key halves, the next group's
+    // reads in flight while one is multiplied (left to itself the compiler
+    // waits for each read before its product); the halves alternate, so no
+    // product waits for the one before it
+    constexpr int KH = KS / 2;
+    u32x4 ka[2][2][KH];
+    auto read = [&](int g) {
 #pragma unroll
-    for (int t = 0; t < 2; ++t)
+      for (int ks = 0; ks < KH; ++ks)
 #pragma unroll
-      for (int i = 0; i < 16; ++i) s[t][i] = 0.f;
+        for (int t = 0; t < 2; ++t)
+          ka[g][t][ks] = *reinterpret_cast<const u32x4*>(
+              kt + (t * 32 + col) * ROWB + ((((g * KH + ks) * 2 + h) ^ (col & (CPR - 1))) << 4));
+    };
+    read(0);
+    read(1);
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int t = 0; t < 2; ++t)
+    for (int g = 0; g < 2; ++g)
 #pragma unroll
-      for (int ks = 0; ks < KS; ++ks) {
-        const int r = t * 32 + col;
-        const u32x4 ka = *reinterpret_cast<const u32x4*>(kt + r * ROWB + (((ks * 2 + h) ^ (r & (CPR - 1))) << 4));
-        s[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_bf16x8(ka), qB[ks], s[t], 0, 0, 0);
-      }
+      for (int ks = 0; ks < KH; ++ks)
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+          s[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+              as_bf16x8(ka[g][t][ks]), qB[g * KH + ks],
+              g == 0 && ks == 0 ? f32x16{0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f} : s[t],
+              0, 0, 0);
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  auto values = [&](int vb, int n0) {  // softmax of the tile's scores, O^T += V^T P^T
+    if (n0 > pos_last) return;  // uniform
+    const unsigned char* vt = lds.vt[vb];
     // lane (h, col), element i of tile t: key n0 + 32 t + 8 (i / 4) + 4 h + i % 4, row col
-    if (n0 + kKeys - 1 > pos_first || holes) {
+    if (n0 + kKeys - 1 > pos_first) {  // uniform: some key lies past the wave's first row
 #pragma unroll
       for (int t = 0; t < 2; ++t)
 #pragma unroll
         for (int i = 0; i < 16; ++i) {
-          const int key = n0 + t * 32 + (i >> 2) * 8 + h * 4 + (i & 3);
-          bool ok = key <= pos;
-          if (holes) ok = ok && lds.pages[(min(key, key_end - 1) >> a.bs_log2) - pg0] >= 0;
-          s[t][i] = ok ? s[t][i] : kNegInf;
+          const int key = t * 32 + (i >> 2) * 8 + h * 4 + (i & 3);
+          s[t][i] = key <= pos - n0 ? s[t][i] : kNegInf;
         }
+    }
+    if (holes) {  // uniform
+      const int key = min(n0 + lane, key_end - 1);
+      const uint64_t mapped = __ballot(lds.pages[(key >> a.bs_log2) - pg0] >= 0) >> (4 * h);
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int i = 0; i < 16; ++i)
+          s[t][i] = (mapped >> (t * 32 + (i >> 2) * 8 + (i & 3))) & 1 ? s[t][i] : kNegInf;
     }
     float mx = fmaxf(s[0][0], s[1][0]);
 #pragma unroll
@@ -227,50 +281,98 @@ __global__ __launch_bounds__(NW * 64, 2) void prefill_attn_kernel(PrefillArgs a)
       m_ref = mn;
     }
     const float nb = m_ref == kNegInf ? 0.f : -m_ref * sc;
-#pragma unroll
-    for (int t = 0; t < 2; ++t) {
-      float sum = 0.f;
-#pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        s[t][i] = __builtin_amdgcn_exp2f(fmaf(s[t][i], sc, nb));
-        sum += s[t][i];
-      }
-      l_run += sum;
-    }
     // O^T += V^T P^T, 16 keys per step: element j of lane half h is key
-    // 8 (j / 4) + 4 h + j % 4 of the step in both operands
-#pragma unroll
-    for (int st = 0; st < kKeys / 16; ++st) {
-      u32x4 pw;
-#pragma unroll
-      for (int e = 0; e < 4; ++e) pw[e] = pack_bf16x2(s[st >> 1][(st & 1) * 8 + 2 * e], s[st >> 1][(st & 1) * 8 + 2 * e + 1]);
-      const bf16x8 pB = as_bf16x8(pw);
+    // 8 (j / 4) + 4 h + j % 4 of the step in both operands.  A step's weights
+    // are computed, and its V operands read, during the step before's products.
+    constexpr int ST = kKeys / 16;
+    uint2 va[2][DT][2];
+    auto read = [&](int st) {
 #pragma unroll
       for (int dt = 0; dt < DT; ++dt) {
         // 16-lane group (h, g): rows 4 h + 0..3 of the step (then + 8), dims 32 dt + 16 g .. + 15
         const int i = lane & 15, g = (lane >> 4) & 1;
-        const int r = st * 16 + h * 4 + (i >> 2);
+        const int r = h * 4 + (i >> 2);
         const int X = dt * 4 + g * 2 + ((i & 3) >> 1);
-        const unsigned char* src = vt + r * ROWB + ((X ^ vswz(r)) << 4) + (i & 1) * 8;
-        const uint2 lo = lds_read_tr(src);
-        const uint2 hi = lds_read_tr(src + 8 * ROWB);  // (vswz(r + 8) == vswz(r))
-        const bf16x8 vA = as_bf16x8(u32x4{lo.x, lo.y, hi.x, hi.y});
-        acc[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vA, pB, acc[dt], 0, 0, 0);
+        const unsigned char* src = vt + r * ROWB + ((X ^ vswz(r)) << 4) + (i & 1) * 8 + st * 16 * ROWB;
+        va[st & 1][dt][0] = lds_read_tr(src);  // (vswz(r + 8) == vswz(r))
+        va[st & 1][dt][1] = lds_read_tr(src + 8 * ROWB);
       }
+    };
+    bf16x8 pB[2];
+    auto weights = [&](int st) {
+      u32x4 pw;
+      float sum = 0.f;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const float p0 = __builtin_amdgcn_exp2f(fmaf(s[st >> 1][(st & 1) * 8 + 2 * e], sc, nb));
+        const float p1 = __builtin_amdgcn_exp2f(fmaf(s[st >> 1][(st & 1) * 8 + 2 * e + 1], sc, nb));
+        sum += p0 + p1;
+        pw[e] = pack_bf16x2(p0, p1);
+      }
+      l_run += sum;
+      pB[st & 1] = as_bf16x8(pw);
+    };
+    read(0);
+    weights(0);
+#pragma unroll
+    for (int st = 0; st < ST; ++st) {
+      if (st + 1 < ST) {
+        read(st + 1);
+        weights(st + 1);
+      }
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt) {
+        const uint2 lo = va[st & 1][dt][0], hi = va[st & 1][dt][1];
+        acc[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_bf16x8(u32x4{lo.x, lo.y, hi.x, hi.y}), pB[st & 1], acc[dt], 0, 0, 0);
+      }
+      __builtin_amdgcn_sched_barrier(0);
     }
   };
 
   if (key_end > key_begin) {  // (uniform; a paged part past the table's last key has none)
-    issue(key_begin);
-    stage(0, key_begin);
+    const int last = key_begin + (key_end - 1 - key_begin) / kKeys * kKeys;  // the last tile's first key
+    issue(0, 0, key_begin);
+    if (DIST == 2 && key_begin < last) issue(1, 1, key_begin + kKeys);
+    // (the query operands are waited for here: a wait for them inside the loop
+    // would wait for the tiles loading ahead)
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) __asm__ volatile("" ::"v"(__builtin_bit_cast(u32x4, qB[ks])));
+    landed(key_begin < last);
     lds_barrier();
-    int buf = 0;
-    for (int n0 = key_begin; n0 < key_end; n0 += kKeys, buf ^= 1) {
-      const bool more = n0 + kKeys < key_end;
-      if (more) issue(n0 + kKeys);
-      compute(buf, n0);
-      if (more) stage(buf ^ 1, n0 + kKeys);
-      lds_barrier();
+    // The upper waves of the 8 (one of each SIMD's two) run half a tile
+    // behind: the softmax of their tile falls into the lower waves' matrix
+    // products and back.  Their V tile stays staged one step longer.
+    auto next = [](int x, int n) { return x + 1 == n ? 0 : x + 1; };
+    int kb = 0, vb = 0, kf = DIST % KB, vf = DIST % VB;  // this tile's buffers, and those of the tile issued beside it
+    auto advance = [&]() {
+      kb = next(kb, KB);
+      vb = next(vb, VB);
+      kf = next(kf, KB);
+      vf = next(vf, VB);
+    };
+    if (!SKEW || w < NW / 2) {
+      for (int n0 = key_begin; n0 <= last; n0 += kKeys) {
+        const int nf = n0 + DIST * kKeys;
+        if (nf <= last) issue(kf, vf, nf);
+        scores(kb, n0);
+        values(vb, n0);
+        landed(nf <= last);
+        lds_barrier();
+        advance();
+      }
+    } else {
+      int vp = 0;
+      for (int n0 = key_begin; n0 <= last; n0 += kKeys) {
+        const int nf = n0 + DIST * kKeys;
+        if (nf <= last) issue(kf, vf, nf);
+        if (n0 > key_begin) values(vp, n0 - kKeys);
+        scores(kb, n0);
+        vp = vb;
+        landed(nf <= last);
+        lds_barrier();
+        advance();
+      }
+      values(vp, last);
     }
   }
 
