@@ -201,9 +201,25 @@ __device__ __forceinline__ int num_splits(const VerifyArgs& a, int ctx) {
   return ctx <= len ? 1 : (ctx + len - 1) / len;
 }
 
+// The key-split kernel's automatic splits are counted by the context at hand
+// (the host's plan knows only the table's width): more than 8 (a merge of
+// more than one round trip) only while they are at least 512 keys long, at
+// most 4 up to 512 keys, and one (no merge at all) up to 320 keys, 200 for
+// one 16-row tile of query rows, whose merge is cheaper.  Measured at 8 pairs
+// and 18 rows, us per call (plan's even splits -> these): 17-page table
+// (9 splits) 100 keys 8.9 -> 6.3, 300 9.0 -> 8.0, 400 9.1 -> 8.5, 1,250 12.3
+// -> 10.2, 4,200 16.1 -> 14.5; 130-page table (32 splits) 1,250 keys 18.4 ->
+// 10.2, 9,000 24.6 -> 21.3; 64 pairs (4 splits) 100 keys 8.4 -> 6.8; two
+// splits at 300 keys instead of one 9.0; 4 rows, one tile, 300 keys: one
+// split 7.0 against 6.8 for eight.
+template <int MT>
 __device__ __forceinline__ int split_len_ks(const VerifyArgs& a, int ctx) {
   if (a.split_tokens > 0) return a.split_tokens;
-  const int per = div_small(ctx + a.ks_splits - 1, a.ks_splits);
+  int n = a.ks_splits;
+  if (n > 8) n = max(8, min(n, ctx >> 9));
+  if (MT > 1 && ctx <= 512) n = min(n, 4);
+  if (ctx <= (MT > 1 ? 320 : 200)) n = 1;
+  const int per = div_small(ctx + n - 1, n);
   return per <= 16 ? 16 : (per + 15) & ~15;
 }
 __device__ __forceinline__ int num_splits_ks(int ctx, int len) { return ctx <= len ? 1 : div_small(ctx + len - 1, len); }
@@ -1008,7 +1024,7 @@ __global__ __launch_bounds__(NW * 64, 8 / NW) void verify_attn_ks_kernel(VerifyA
   if (pair_raw >= a.npairs) return;
   const int ctx = clamp_context(a, ctx_raw);
   const int qlen = q1 - q0;
-  const int len = split_len_ks(a, ctx);
+  const int len = split_len_ks<MT>(a, ctx);
   const int nsplit = num_splits_ks(ctx, len);
   if (split >= nsplit || qlen < 0) return;  // uniform per workgroup
   const int kb = split * len;

@@ -256,3 +256,16 @@ def test_fp32_tile_edges(G, ql, D, bs):
         vb.block_tables[8, 2] = -1
     out = _gpu(vb, max_q_len=ql)
     assert_close(out, _oracle(vb), "f32", "fp32 edges")
+
+
+@pytest.mark.parametrize("G,ql", [(2, 1), (2, 9), (4, 9)])
+def test_split_counts_follow_the_context(G, ql):
+    # a 10k-key table plans more than 8 splits; the kernel counts a context's
+    # splits by its own length: the lengths around each change of the rule,
+    # for one, two and three row tiles, short and long contexts in one call
+    print(f"case: splits by context, {G} heads x {ql} rows", flush=True)
+    ctx = [9, 100, 200, 201, 320, 321, 512, 513, 4607, 4608, 5121, 1250]
+    vb = synth.verify_batch(43, ctx, [ql] * len(ctx), num_heads=2 * G, num_kv_heads=2, dtype="bf16", max_blocks=40)
+    assert _kernel(vb, ql) == "key-split"
+    out = _gpu(vb, max_q_len=ql)
+    assert_close(out, _oracle(vb), "bf16", "splits by context")
