@@ -121,6 +121,20 @@ int nsv_prefill_attention(void* out, const void* q, const void* k,
                           int max_blocks, void* partials, void* stream);
 
 /*
+ * The work list of nsv_prefill_attention for n sequences of seqlens_q[b] new
+ * rows that end seqlens_k[b] keys each (host arrays; 0 < seqlens_q <=
+ * seqlens_k), on a device with `cus` compute units.  block_size 0: contiguous
+ * K/V, the sequences' keys back to back.  Writes the tiles [ntiles, 8] and
+ * behind them the merges [nmerges, 4] to `out` (host memory, `capacity`
+ * words) and to counts[4] the two counts, tile_rows and the partial slots;
+ * NSV_ERR_WORKSPACE with the counts set when `capacity` is too small.
+ * Host-only, launches nothing.
+ */
+int nsv_prefill_tiles(const int64_t* seqlens_q, const int64_t* seqlens_k,
+                      int n, int H, int Hkv, int block_size, int cus,
+                      int32_t* out, int64_t capacity, int32_t* counts);
+
+/*
  * Load-only measurement kernels, no reference counterpart (the ceilings
  * against which bench.py --ceiling reads the verify-attention kernels).
  * nsv_verify_attention_load_floor reads exactly the K/V bytes of a bf16,

@@ -41,6 +41,7 @@ SIGNATURES: dict[str, tuple] = {
     "nsv_verify_attention_noalloc": (
         _c_int,
         [_c_vp] * 8 + [_c_f32] + [_c_int] * 10 + [_c_vp]),
+    "nsv_prefill_tiles": (_c_int, [_c_vp] * 2 + [_c_int] * 5 + [_c_vp, _c_i64, _c_vp]),
     "nsv_prefill_attention": (
         _c_int, [_c_vp] * 6 + [_c_int] * 2 + [_c_vp, _c_int, _c_f32] + [_c_int] * 5 + [_c_vp] * 2),
     "nsv_verify_attention_load_floor": (_c_int, [_c_vp] * 4 + [_c_int] * 6 + [_c_vp, _c_vp]),

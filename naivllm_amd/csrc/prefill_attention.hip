@@ -31,6 +31,11 @@
 
 #include "common.h"
 
+#include <algorithm>
+#include <array>
+#include <new>
+#include <vector>
+
 namespace {
 
 typedef float f32x16 __attribute__((ext_vector_type(16)));
@@ -459,9 +464,105 @@ __global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillMergeArgs a) 
       make_uint2(pack_bf16x2(num[0] * inv, num[1] * inv), pack_bf16x2(num[2] * inv, num[3] * inv));
 }
 
+// ---------------------------------------------------------------------------
+// The work list (host).  Rows per tile: a workgroup of 8 waves of 32 rows
+// (two query heads of a kv head where the group is even) reads a K/V tile for
+// twice the rows of a 4-wave one, but fewer, larger workgroups fill the chip
+// worse and idle longer at the causal edge.  Measured on MI355X, 4 against 8
+// waves: 8 prompts of ~1000 tokens (16/8 heads) 59 against 70 us, one of 1206
+// 36 against 40, 4096 (32/8 heads) 171 against 148, two of 2900-4050 behind
+// 4096 cached keys 800 against 725: 8 waves from 24 key tiles per tile on
+// average.
+//
+// Cut over keys: where the tiles alone are fewer than the compute units, a
+// tile's chain of key tiles (~1.8 us each with one wave per SIMD) is the
+// call's time, so tiles longer than 1.5 targets are cut into parts of about
+// `target` key tiles and merged by a second kernel: 40 rows behind 4096 keys
+// 114 -> 20 us (targets 3 and 4; 6: 21, 8: 24), 270 rows of 32/8 heads 120 ->
+// 50-62 (16, 12), one prompt of 1206 40 -> 31 (4; 3: 35, 8: 34).  With more
+// tiles than compute units the partials cost what the shorter chain saves
+// (1206 of 32/8 heads, 304 workgroups: 41.7 -> 39-43; 8 prompts 59 ->
+// 64-172), so those stay whole.
+// ---------------------------------------------------------------------------
+struct Tiling {
+  std::vector<std::array<int32_t, kTileWords>> tiles;
+  std::vector<std::array<int32_t, 4>> merges;
+  int rows, slots;
+};
+
+Tiling make_tiles(const int64_t* ql, const int64_t* kl, int n, int H, int Hkv, int block_size, int cus) {
+  const int hw = (H / Hkv) % 2 == 0 ? 2 : 1;
+  auto key_tiles = [](int64_t end) { return (end + kKeys - 1) / kKeys; };
+  auto count = [&](int rows, int64_t& tiles, int64_t& keys) {
+    tiles = keys = 0;
+    for (int b = 0; b < n; ++b)
+      for (int64_t r = 0; r < ql[b]; r += rows) {
+        ++tiles;
+        keys += key_tiles(kl[b] - ql[b] + std::min(r + rows, ql[b]));
+      }
+  };
+  Tiling t{{}, {}, 8 * kWaveRows / hw, 0};
+  int64_t tiles, keys;
+  count(t.rows, tiles, keys);
+  if (keys < 24 * tiles) {
+    t.rows /= 2;
+    count(t.rows, tiles, keys);
+  }
+  const int64_t units = H / hw;  // workgroups per tile
+  const int64_t target = std::max<int64_t>(4, (keys * units * 2 + 3 * cus - 1) / (3 * cus));
+  const int64_t most = std::max<int64_t>(1, (int64_t)(kMaxPages - 1) * block_size / kKeys);  // a part's pages fit LDS
+  t.tiles.reserve(tiles);
+  int64_t q0 = 0, k0 = 0;
+  for (int b = 0; b < n; ++b) {
+    for (int64_t r = 0; r < ql[b]; r += t.rows) {
+      const int64_t nr = std::min<int64_t>(t.rows, ql[b] - r), pos = kl[b] - ql[b] + r, end = pos + nr, nt = key_tiles(end);
+      int64_t parts = tiles * units <= cus && 2 * nt > 3 * target ? (nt + target - 1) / target : 1;
+      if (block_size > 0) parts = std::max(parts, (nt + most - 1) / most);
+      const int64_t per = (nt + parts - 1) / parts;
+      parts = (nt + per - 1) / per;
+      if (parts > 1) t.merges.push_back({t.slots, (int32_t)parts, (int32_t)(q0 + r), (int32_t)nr});
+      for (int64_t i = 0; i < parts; ++i)
+        t.tiles.push_back({b, (int32_t)(q0 + r), (int32_t)nr, (int32_t)pos, (int32_t)(block_size > 0 ? 0 : k0),
+                           (int32_t)(i * per * kKeys), (int32_t)std::min(end, (i + 1) * per * kKeys),
+                           parts > 1 ? t.slots++ : -1});
+    }
+    q0 += ql[b];
+    k0 += kl[b];
+  }
+  std::stable_sort(t.tiles.begin(), t.tiles.end(),
+                   [](const auto& x, const auto& y) { return x[6] - x[5] > y[6] - y[5]; });  // heaviest first
+  return t;
+}
+
 }  // namespace
 
 extern "C" {
+
+int nsv_prefill_tiles(const int64_t* seqlens_q, const int64_t* seqlens_k, int n, int H, int Hkv, int block_size,
+                      int cus, int32_t* out, int64_t capacity, int32_t* counts) {
+  if (n < 0 || H <= 0 || Hkv <= 0 || H % Hkv || block_size < 0 || cus <= 0 || capacity < 0 || !counts) return NSV_ERR_ARG;
+  if (n > 0 && (!seqlens_q || !seqlens_k || !out)) return NSV_ERR_ARG;
+  int64_t rows = 0, keys = 0;
+  for (int b = 0; b < n; ++b) {
+    if (seqlens_q[b] <= 0 || seqlens_q[b] > seqlens_k[b] || seqlens_k[b] > ((int64_t)1 << 30)) return NSV_ERR_ARG;
+    rows += seqlens_q[b];
+    keys += seqlens_k[b];
+  }
+  if (rows > 0x7fffffff || keys > 0x7fffffff) return NSV_ERR_UNSUPPORTED;
+  try {
+    const Tiling t = make_tiles(seqlens_q, seqlens_k, n, H, Hkv, block_size, cus);
+    counts[0] = (int32_t)t.tiles.size();
+    counts[1] = (int32_t)t.merges.size();
+    counts[2] = t.rows;
+    counts[3] = t.slots;
+    if ((int64_t)t.tiles.size() * kTileWords + (int64_t)t.merges.size() * 4 > capacity) return NSV_ERR_WORKSPACE;
+    for (const auto& x : t.tiles) out = std::copy(x.begin(), x.end(), out);
+    for (const auto& x : t.merges) out = std::copy(x.begin(), x.end(), out);
+  } catch (const std::bad_alloc&) {
+    return NSV_ERR_WORKSPACE;
+  }
+  return NSV_OK;
+}
 
 int nsv_prefill_attention(void* out, const void* q, const void* k, const void* v, const int32_t* block_tables,
                           const int32_t* tiles, int ntiles, int tile_rows, const int32_t* merges, int nmerges,

@@ -9,6 +9,8 @@ PyTorch fallback.
 
 from __future__ import annotations
 
+import ctypes
+
 import torch
 import torch.nn as nn
 
@@ -55,7 +57,6 @@ def verify_attention_plan(batch_size: int, num_heads: int, num_kv_heads: int, he
                           cus: int = 0) -> tuple[str, int]:
     """(kernel, key splits per sequence) that paged_attention_verify runs for
     this shape on a device with ``cus`` compute units (0: the current one)."""
-    import ctypes
     kind, splits = ctypes.c_int(), ctypes.c_int()
     rc = _lib.lib().nsv_verify_attention_plan(batch_size, num_heads, num_kv_heads, head_dim, block_size,
                                              max_num_blocks, max_q_len, _lib.dtype_code(dtype), kv_split_tokens,
@@ -183,94 +184,52 @@ def store_kvcache(
     _lib.check(rc, "store_kvcache")
 
 
-_PREFILL_KEYS = 64    # keys per tile of the prefill kernel
-_PREFILL_PAGES = 2048  # block-table entries it stages for one record
+def _prefill_work(seqlens_q, seqlens_k, num_heads: int, num_kv_heads: int, block_size: int | None, cus: int,
+                  pinned: bool) -> tuple[torch.Tensor, list[int]]:
+    """nsv_prefill_tiles into a host tensor; returns (its words, [tiles,
+    merges, tile_rows, slots])."""
+    seqlens_q, seqlens_k = [int(x) for x in seqlens_q], [int(x) for x in seqlens_k]
+    n = len(seqlens_q)
+    if n != len(seqlens_k):
+        raise ValueError("seqlens_q and seqlens_k differ in length")
+    for i, (ql, kl) in enumerate(zip(seqlens_q, seqlens_k)):
+        if not 0 < ql <= kl:
+            raise ValueError(f"prefill sequence {i}: {ql} query rows over {kl} keys")
+    q, k, counts = (ctypes.c_int64 * n)(*seqlens_q), (ctypes.c_int64 * n)(*seqlens_k), (ctypes.c_int32 * 4)()
+    words = 4096
+    while True:
+        buf = torch.empty(words, dtype=torch.int32, pin_memory=pinned)
+        rc = _lib.lib().nsv_prefill_tiles(q, k, n, num_heads, num_kv_heads, block_size or 0, cus, buf.data_ptr(),
+                                          words, counts)
+        need = 8 * counts[0] + 4 * counts[1]
+        if rc == 0 or need <= words:
+            break
+        words = need
+    _lib.check(rc, "prefill_tiles")
+    return buf[:need], list(counts)
 
 
 def prefill_tiles(seqlens_q, seqlens_k, num_heads: int, num_kv_heads: int, block_size: int | None, cus: int):
-    """The prefill kernel's work list (nsv_prefill_attention) for sequences of
-    seqlens_q new rows ending seqlens_k keys each; block_size None: K/V are
-    the sequences' keys back to back.  Host arithmetic only.
-    Returns (tiles [n, 8] int32, merges [m, 4] int32, tile_rows, slots).
-
-    Rows per tile: a workgroup of 8 waves of 32 rows (two query heads of a kv
-    head where the group is even) reads a K/V tile for twice the rows of a
-    4-wave one, but fewer, larger workgroups fill the chip worse and idle
-    longer at the causal edge.  Measured on MI355X, 4 against 8 waves: 8
-    prompts of ~1000 tokens (16/8 heads) 59 against 73 us, one of 1206 39
-    against 45, 4096 (32/8 heads) 180 against 161, two of 2900-4050 behind
-    4096 cached keys 870 against 781: 8 waves from 24 key tiles per record on
-    average.
-
-    Cut over keys: where the tiles alone are fewer than the compute units, a
-    record's chain of key tiles (~1.8 us each with one wave per SIMD) is the
-    call's time, so tiles longer than 1.5 targets are cut into parts of about
-    `target` key tiles and merged by a second kernel: 40 rows behind 4096
-    keys 114 -> 20 us (targets 3 and 4; 6: 21, 8: 24), 270 rows of 32/8 heads
-    120 -> 50-62 (16, 12), one prompt of 1206 40 -> 31 (4; 3: 35, 8: 34).
-    With more tiles than compute units the partials cost what the shorter
-    chain saves (1206 of 32/8 heads, 304 workgroups: 41.7 -> 39-43; 8 prompts
-    59 -> 64-172), so those stay whole."""
-    import numpy as np
-
-    ql, kl = np.asarray(seqlens_q, dtype=np.int64), np.asarray(seqlens_k, dtype=np.int64)
-    if len(ql) != len(kl):
-        raise ValueError("seqlens_q and seqlens_k differ in length")
-    bad = np.nonzero((ql <= 0) | (ql > kl))[0]
-    if len(bad):
-        raise ValueError(f"prefill sequence {bad[0]}: {ql[bad[0]]} query rows over {kl[bad[0]]} keys")
-    group = num_heads // num_kv_heads
-    hw = 2 if group % 2 == 0 else 1
-    q0, k0 = np.cumsum(ql) - ql, np.cumsum(kl) - kl
-
-    def cut(rows):
-        n = -(-ql // rows)  # tiles per sequence
-        seq = np.repeat(np.arange(len(ql)), n)
-        first = (np.arange(len(seq)) - np.repeat(np.cumsum(n) - n, n)) * rows  # first new row of the tile
-        nr = np.minimum(rows, ql[seq] - first)
-        pos = kl[seq] - ql[seq] + first
-        return seq, q0[seq] + first, nr, pos, -(-(pos + nr) // _PREFILL_KEYS)
-
-    rows = 8 * 32 // hw
-    seq, row0, nr, pos, nt = cut(rows)
-    if nt.sum() < 24 * len(nt):
-        rows //= 2
-        seq, row0, nr, pos, nt = cut(rows)
-    units = len(seq) * (num_heads // hw)
-    parts = np.ones_like(nt)
-    if units <= cus:
-        target = max(4, -(-int(nt.sum()) * (num_heads // hw) * 2 // (3 * cus)))
-        parts = np.where(2 * nt > 3 * target, -(-nt // target), parts)
-    if block_size is not None:  # a record's pages fit the kernel's LDS copy
-        parts = np.maximum(parts, -(-nt // max(1, (_PREFILL_PAGES - 1) * block_size // _PREFILL_KEYS)))
-    per = -(-nt // parts)
-    parts = -(-nt // per)
-    slot0 = np.cumsum(np.where(parts > 1, parts, 0)) - np.where(parts > 1, parts, 0)
-    cuts = parts > 1
-    merges = np.stack([slot0[cuts], parts[cuts], row0[cuts], nr[cuts]], axis=1).astype(np.int32)
-    t = np.repeat(np.arange(len(seq)), parts)  # the tile of each record
-    i = np.arange(len(t)) - np.repeat(np.cumsum(parts) - parts, parts)
-    begin = i * per[t] * _PREFILL_KEYS
-    end = np.minimum(pos[t] + nr[t], begin + per[t] * _PREFILL_KEYS)
-    kv0 = k0[seq[t]] if block_size is None else np.zeros_like(t)
-    tiles = np.stack([seq[t], row0[t], nr[t], pos[t], kv0, begin, end, np.where(cuts[t], slot0[t] + i, -1)], axis=1)
-    order = np.argsort(begin - end, kind="stable")  # heaviest first
-    return tiles[order].astype(np.int32), merges, rows, int(parts[cuts].sum())
+    """The prefill kernel's work list for sequences of seqlens_q new rows
+    ending seqlens_k keys each (nsv_prefill_tiles); block_size None: K/V are
+    the sequences' keys back to back.  Host only.
+    Returns (tiles [n, 8] int32, merges [m, 4] int32, tile_rows, slots)."""
+    work, (nt, nm, rows, slots) = _prefill_work(seqlens_q, seqlens_k, num_heads, num_kv_heads, block_size, cus, False)
+    return work[:8 * nt].view(nt, 8).numpy(), work[8 * nt:].view(nm, 4).numpy(), rows, slots
 
 
 class PrefillPlan:
     """The work list of one prefill step on the device, in one transfer."""
 
     def __init__(self, seqlens_q, seqlens_k, num_heads: int, num_kv_heads: int, block_size: int | None, device):
-        import numpy as np
-
         cus = torch.cuda.get_device_properties(device).multi_processor_count
-        tiles, merges, self.tile_rows, self.slots = prefill_tiles(seqlens_q, seqlens_k, num_heads, num_kv_heads,
-                                                                  block_size, cus)
+        # (as _lib.upload: not waited for, except inside a capture, which refuses the wait)
+        ahead = not torch.cuda.is_current_stream_capturing()
+        work, (self.ntiles, self.nmerges, self.tile_rows, self.slots) = _prefill_work(
+            seqlens_q, seqlens_k, num_heads, num_kv_heads, block_size, cus, ahead)
         self.num_heads, self.num_kv_heads, self.block_size = num_heads, num_kv_heads, block_size
         self.sequences, self.rows, self.keys = len(seqlens_q), int(sum(seqlens_q)), int(sum(seqlens_k))
-        self.ntiles, self.nmerges = len(tiles), len(merges)
-        self.work = _lib.upload(np.concatenate([tiles.ravel(), merges.ravel()]), device)
+        self.work = work.to(device, non_blocking=ahead)
 
 
 def prefill_attention(query: torch.Tensor, k: torch.Tensor, v: torch.Tensor, plan: PrefillPlan, scale: float,
