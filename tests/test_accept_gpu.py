@@ -456,3 +456,25 @@ def test_unaligned_rows(dtype, V):
     qn = torch.empty(B, V, device="cuda").exponential_(1, generator=torch.Generator(device="cuda").manual_seed(114))
     qn.clamp_min_(1e-10)
     assert sample(rows, temps, qn).tolist() == oa.sample_rows(host(rows), temps.cpu().numpy(), qn.cpu().numpy())
+
+
+@pytest.mark.parametrize("dtype", ["bf16", "f32"])
+@pytest.mark.parametrize("V", [2, 7, 8, 9, 2047, 2048, 2049, 4105])
+def test_resample_rows_around_groups_and_chunks(dtype, V):
+    # resampled rows whose stored residuals end inside an 8-element group or at
+    # a 2048-element chunk, several sequences' rows behind one another; a
+    # uniform of 1 rejects unless the ratio is above it
+    print(f"case: resample rows {dtype} V={V}", flush=True)
+    B, K = 5, 2
+    dl, tl = logits_tensor(81, B * K, V, dtype), logits_tensor(82, B * (K + 1), V, dtype)
+    lists = [[int(x) for x in synth.randint(b + V, 83, K, 0, V)] for b in range(B)]
+    u, q = draw_randomness([K] * B, V, TDT[dtype], "cuda", True, torch.Generator(device="cuda").manual_seed(V))
+    u[:, 0] = torch.tensor([1.0, 0.0, 1.0, 0.5, 1.0], device="cuda")
+    d, nd = pad(lists, K)
+    got = results(*accept_stochastic(tl, d, nd, torch.ones(B, device="cuda"), q, uniforms=u, draft_logits=dl,
+                                     target_seq_stride=K + 1, draft_seq_stride=K, draft_row_stride=1))
+    T, D, U, Q = host(tl), host(dl), u.cpu().numpy(), host(q)
+    for b in range(B):
+        want = oa.verify_stochastic(lists[b], T[b * (K + 1):(b + 1) * (K + 1)], D[b * K:(b + 1) * K], 1.0, U[b], Q[b],
+                                    dtype)
+        assert got[b] == want, (b, got[b], want)
