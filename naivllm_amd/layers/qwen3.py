@@ -179,6 +179,23 @@ def wide_splits(M: int, N: int, K: int, swiglu: bool = False, packed: bool = Fal
     return int(_lib.lib().nsv_wide_linear_splits(M, N, K, int(swiglu), int(packed)))
 
 
+def dense_bf16(t: torch.Tensor | None, M: int, N: int, device) -> bool:
+    """Whether t is what the projections write: contiguous bf16 [M, N] on device."""
+    return (t is not None and tuple(t.shape) == (M, N) and t.dtype == torch.bfloat16 and t.is_contiguous()
+            and t.device == device)
+
+
+def _check_partials(partials: torch.Tensor | None, splits: int, T: int, N: int, device) -> None:
+    if (partials is None or partials.dtype != torch.float32 or not partials.is_contiguous()
+            or partials.device != device or partials.numel() < splits * T * N):
+        raise ValueError(f"partials: contiguous fp32 of at least {splits} x {T} x {N} on {device}")
+
+
+def _check_cuda(t: torch.Tensor, what: str) -> None:
+    if not t.is_cuda:
+        raise ValueError(f"{what} runs on the GPU; its input is on {t.device}")
+
+
 def wide_linear(x: torch.Tensor, weight: torch.Tensor, y: torch.Tensor | None, partials: torch.Tensor | None = None, *,
                 swiglu: bool = False, packed: bool = False) -> None:
     """y = x @ weight.T on the weight-streaming kernel of up to 128 rows
@@ -188,9 +205,16 @@ def wide_linear(x: torch.Tensor, weight: torch.Tensor, y: torch.Tensor | None, p
     packed layout."""
     M, K = x.shape
     N = weight.shape[0]
-    if weight.shape[1] != K or not (x.is_contiguous() and weight.is_contiguous()):
-        raise ValueError(f"wide_linear: x [M, K] and weight [N, K], contiguous; got {tuple(x.shape)}, "
-                         f"{tuple(weight.shape)}")
+    if (weight.shape[1] != K or not (x.is_contiguous() and weight.is_contiguous())
+            or not (x.dtype == weight.dtype == torch.bfloat16)):
+        raise ValueError(f"wide_linear: x [M, K] and weight [N, K], contiguous bf16; got {tuple(x.shape)} {x.dtype}, "
+                         f"{tuple(weight.shape)} {weight.dtype}")
+    splits = wide_splits(M, N, K, swiglu, packed)
+    if splits > 1:
+        _check_partials(partials, splits, M, N, x.device)
+    elif not dense_bf16(y, M, N // 2 if swiglu else N, x.device):
+        raise ValueError(f"wide_linear: y must be a contiguous bf16 [{M}, {N // 2 if swiglu else N}] on {x.device}")
+    _check_cuda(x, "wide_linear")
     rc = _lib.lib().nsv_wide_linear(x.data_ptr(), weight.data_ptr(), _lib.ptr(y), _lib.ptr(partials), M, N, K,
                                     int(swiglu), int(packed), _lib.stream_ptr(x.device))
     _lib.check(rc, "wide_linear")
@@ -200,6 +224,11 @@ def rms_norm_sum(partials: torch.Tensor, splits: int, weight: torch.Tensor, eps:
                  residual: torch.Tensor, residual_out: torch.Tensor | None = None) -> None:
     """rms_norm whose x is the sum of a split projection's partials."""
     T, E = out.shape
+    _check_partials(partials, splits, T, E, out.device)
+    if (not all(dense_bf16(t, T, E, out.device) for t in (out, residual, residual if residual_out is None else residual_out))
+            or tuple(weight.shape) != (E,) or weight.dtype != torch.bfloat16):
+        raise ValueError(f"rms_norm_sum: out, residual and residual_out [{T}, {E}] and weight [{E}], contiguous bf16")
+    _check_cuda(out, "rms_norm_sum")
     rc = _lib.lib().nsv_rms_norm_sum(partials.data_ptr(), splits, residual.data_ptr(), _lib.ptr(residual_out),
                                      weight.data_ptr(), out.data_ptr(), T, E, eps, _lib.stream_ptr(out.device))
     _lib.check(rc, "rms_norm_sum")
@@ -210,6 +239,11 @@ def qk_norm_rope_store_sum(partials, splits: int, q_norm_w, k_norm_w, rope_rows,
     """qk_norm_rope_store (one rotary row per step row) whose qkv is the sum
     of a split projection's partials."""
     T = q_out.shape[0]
+    _check_partials(partials, splits, T, (H + 2 * Hkv) * D, q_out.device)
+    if not (rope_rows.shape[0] >= T and slot_mapping.numel() >= T and rope_rows.is_contiguous()
+            and rope_rows.dtype == torch.float32 and slot_mapping.dtype == torch.int64 and slot_mapping.is_contiguous()):
+        raise ValueError(f"qk_norm_rope_store_sum: fp32 rope_rows and int64 slot_mapping of {T} rows, contiguous")
+    _check_cuda(q_out, "qk_norm_rope_store_sum")
     rc = _lib.lib().nsv_qk_norm_rope_store_sum(
         partials.data_ptr(), splits, q_norm_w.data_ptr(), k_norm_w.data_ptr(), rope_rows.data_ptr(),
         slot_mapping.data_ptr(), q_out.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), T, H, Hkv, D, eps,
@@ -356,6 +390,7 @@ class Qwen3Verify:
             self.lm_head_packed = torch.empty_like(self.lm_head)
             _lib.check(_lib.lib().nsv_lm_head_pack(self.lm_head.data_ptr(), self.lm_head_packed.data_ptr(), V, E,
                                                    _lib.stream_ptr(self.device)), "lm_head_pack")
+
     def prefill_q_block(self) -> int:
         """Query rows per causal block of a prefill: the verify kernel serves
         up to 64 (GQA group x rows) per (sequence, kv head)."""
@@ -525,9 +560,13 @@ class Qwen3Verify:
             else:
                 linear(h, self.lm_head, logits_out)
             return logits_out
-        if self.lm_head_packed is not None and T <= WIDE_ROWS and wide_splits(T, *self.lm_head.shape, packed=True):
+        # (a logits_out that the kernel cannot write, a strided view above all,
+        # is left to matmul, which writes it or refuses it)
+        V = self.lm_head.shape[0]
+        if (self.lm_head_packed is not None and T <= WIDE_ROWS and wide_splits(T, V, E, packed=True)
+                and (logits_out is None or dense_bf16(logits_out, T, V, h.device))):
             if logits_out is None:
-                logits_out = torch.empty(T, self.lm_head.shape[0], dtype=self.dtype, device=self.device)
+                logits_out = torch.empty(T, V, dtype=self.dtype, device=self.device)
             wide_linear(h, self.lm_head_packed, logits_out, packed=True)
             return logits_out
         if logits_out is None:

@@ -1,0 +1,63 @@
+"""What the weight-streaming projections and the kernels that sum their
+partials refuse, on the CPU: every buffer they write or read is checked before
+the library is called."""
+
+import pytest
+import torch
+
+import naivllm_amd.layers.qwen3 as qm
+
+BF, F32 = torch.bfloat16, torch.float32
+
+
+def z(*shape, dtype=BF):
+    return torch.zeros(*shape, dtype=dtype)
+
+
+M, N, K = 20, 1024, 256      # one split: y is written
+SN, SK = 1024, 4096          # split: partials are written
+
+
+def test_shapes_are_on_both_sides_of_the_split():
+    assert qm.wide_splits(M, N, K) == 1 and qm.wide_splits(M, SN, SK) > 1
+
+
+@pytest.mark.parametrize("y", [None, z(M, N, dtype=F32), z(M - 1, N), z(M, N - 16), z(M, 2 * N)[:, :N], z(M * N)])
+def test_output_that_the_kernel_cannot_write(y):
+    with pytest.raises(ValueError, match="y must be"):
+        qm.wide_linear(z(M, K), z(N, K), y)
+
+
+def test_swiglu_output_is_half_as_wide():
+    with pytest.raises(ValueError, match="y must be"):
+        qm.wide_linear(z(M, K), z(N, K), z(M, N), swiglu=True)
+
+
+@pytest.mark.parametrize("x,w", [(z(M, K, dtype=F32), z(N, K)), (z(M, K), z(N, K, dtype=F32)), (z(K, M).t(), z(N, K))])
+def test_operands(x, w):
+    with pytest.raises(ValueError, match="contiguous bf16"):
+        qm.wide_linear(x, w, z(M, N))
+
+
+@pytest.mark.parametrize("scale,dtype", [(None, F32), (1, BF), (0.5, F32)])
+def test_partials_of_a_split_projection(scale, dtype):
+    splits = qm.wide_splits(M, SN, SK)
+    part = None if scale is None else z(int(splits * M * SN * scale), dtype=dtype)
+    with pytest.raises(ValueError, match="partials"):
+        qm.wide_linear(z(M, SK), z(SN, SK), None, part)
+    if part is not None:
+        with pytest.raises(ValueError, match="partials"):
+            qm.rms_norm_sum(part, splits, z(SN), 1e-6, z(M, SN), z(M, SN))
+        with pytest.raises(ValueError, match="partials"):
+            qm.qk_norm_rope_store_sum(part, splits, z(128), z(128), z(M, 128, dtype=F32), z(M, dtype=torch.int64),
+                                      z(M, 4, 128), z(2, 16, 2, 128), z(2, 16, 2, 128), 4, 2, 128, 1e-6)
+
+
+def test_sum_consumers_check_their_rows():
+    part = z(2 * M * N, dtype=F32)
+    for out, res, w in ((z(M, N), z(M - 1, N), z(N)), (z(M, N), z(M, N), z(N - 1)), (z(M, N), z(M, N, dtype=F32), z(N))):
+        with pytest.raises(ValueError, match="rms_norm_sum"):
+            qm.rms_norm_sum(part, 2, w, 1e-6, out, res)
+    with pytest.raises(ValueError, match="slot_mapping"):
+        qm.qk_norm_rope_store_sum(part, 2, z(128), z(128), z(M, 128, dtype=F32), z(M - 1, dtype=torch.int64),
+                                  z(M, 4, 128), z(2, 16, 2, 128), z(2, 16, 2, 128), 4, 2, 128, 1e-6)

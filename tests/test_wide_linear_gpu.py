@@ -109,3 +109,29 @@ def test_qk_norm_rope_store_of_a_sum(splits):
     qm.qk_norm_rope_store(x.to(torch.bfloat16), qw, kw, rope, None, slots, *want, H, Hkv, D, 1e-6)
     for a, b in zip(got, want):
         assert torch.equal(a, b)
+
+
+def test_head_writes_or_refuses_the_callers_logits():
+    # 96 rows at hidden 1024: past the streaming head's rows, on the packed copy
+    print("case: logits_out of the wide head", flush=True)
+    cfg = qm.Qwen3Config(vocab_size=2048, hidden_size=1024, num_layers=1, num_heads=4, num_kv_heads=2, head_dim=64,
+                         intermediate_size=512, max_position=256)
+    model = qm.Qwen3Verify(cfg, "cuda", seed=3)
+    model.allocate_kv_cache(8, 16)
+    T, V = 96, cfg.vocab_size
+    assert qm.lm_head_rows(1024) < T and model.lm_head_packed is not None
+    i64 = dict(dtype=torch.int64, device="cuda")
+    pos = torch.arange(T, **i64)
+    bt = torch.arange(8, dtype=torch.int32, device="cuda")[None]
+    plan = qm.PrefillPlan([T], [T], 4, 2, 16, torch.device("cuda"))
+    run = lambda out: model.forward(pos % 50, pos, pos, bt, None, None, 0, logits_out=out, prefill=plan)  # noqa: E731
+    want = run(None)
+    dense = torch.empty(T, V, dtype=torch.bfloat16, device="cuda")
+    assert run(dense) is dense and torch.equal(dense, want)
+    wide = torch.full((T, V + 64), 7.0, dtype=torch.bfloat16, device="cuda")
+    got = run(wide[:, :V])  # rows V + 64 apart
+    torch.testing.assert_close(got.float(), want.float(), **BF16)
+    torch.testing.assert_close(wide[:, :V].float(), want.float(), **BF16)
+    assert (wide[:, V:] == 7.0).all()
+    with pytest.raises(RuntimeError):
+        run(torch.empty(T, V, device="cuda"))  # fp32
