@@ -219,7 +219,10 @@ def prefill_tiles(seqlens_q, seqlens_k, num_heads: int, num_kv_heads: int, block
 
 
 class PrefillPlan:
-    """The work list of one prefill step on the device, in one transfer."""
+    """The work list of one prefill step on the device, in one transfer.
+
+    The transfer is enqueued on the stream that is current here and not waited
+    for; a call on another stream waits for it on the device (use_on)."""
 
     def __init__(self, seqlens_q, seqlens_k, num_heads: int, num_kv_heads: int, block_size: int | None, device):
         cus = torch.cuda.get_device_properties(device).multi_processor_count
@@ -230,6 +233,22 @@ class PrefillPlan:
         self.num_heads, self.num_kv_heads, self.block_size = num_heads, num_kv_heads, block_size
         self.sequences, self.rows, self.keys = len(seqlens_q), int(sum(seqlens_q)), int(sum(seqlens_k))
         self.work = work.to(device, non_blocking=ahead)
+        self.stream = torch.cuda.current_stream(device)
+        self.ready = torch.cuda.Event() if ahead else None  # the transfer is done
+        if ahead:
+            self.ready.record(self.stream)
+
+    def use_on(self, stream) -> None:
+        """Order work enqueued on ``stream`` after the transfer, and keep the
+        list's memory until that work is done.  A capture on another stream
+        can hold no wait for an event from outside it, and needs none:
+        torch.cuda.graph waits for the device before it begins, and whoever
+        replays the graph keeps the plan."""
+        if stream == self.stream or torch.cuda.is_current_stream_capturing():
+            return
+        if self.ready is not None:
+            stream.wait_event(self.ready)
+        self.work.record_stream(stream)
 
 
 def prefill_attention(query: torch.Tensor, k: torch.Tensor, v: torch.Tensor, plan: PrefillPlan, scale: float,
@@ -261,8 +280,9 @@ def prefill_attention(query: torch.Tensor, k: torch.Tensor, v: torch.Tensor, pla
         max_blocks = block_tables.shape[1]
     query = query.contiguous()
     out = torch.empty_like(query)
-    # (from the caching allocator on the current stream: calls on several
-    # streams or threads share nothing)
+    # (the plan's list is the only memory that calls on several streams or
+    # threads share, and they only read it)
+    plan.use_on(torch.cuda.current_stream(query.device))
     part = torch.empty(plan.slots * H * plan.tile_rows * (head_dim + 2), dtype=torch.float32,
                        device=query.device) if plan.slots else None
     tiles = plan.work.data_ptr()

@@ -66,3 +66,31 @@ def test_prefill_attention_refuses_bad_shapes():
     for bad in ((q[:3], k, k), (q, k[:3], k[:3]), (q.float(), k, k), (q, k, k[:, :, :64])):
         with pytest.raises(ValueError):
             prefill_attention(*bad, plan, 1.0, 128)
+
+
+def test_a_plan_serves_other_streams_and_captures():
+    # built on one stream while work is queued there, used at once on another,
+    # then inside a capture (its own stream), replayed twice
+    print("case: prefill plan on other streams", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(3)
+    q = torch.randn(200, 2, 128, generator=g, device="cuda").bfloat16()
+    k, v = (torch.randn(200, 1, 128, generator=g, device="cuda").bfloat16() for _ in range(2))
+    want = prefill_attention(q, k, v, PrefillPlan([200], [200], 2, 1, None, q.device), 0.1, 128)
+    busy = torch.zeros(1 << 26, device="cuda")
+    torch.cuda.synchronize()
+    side = torch.cuda.Stream()
+    for _ in range(8):
+        busy.add_(1)
+    plan = PrefillPlan([200], [200], 2, 1, None, q.device)
+    with torch.cuda.stream(side):
+        got = prefill_attention(q, k, v, plan, 0.1, 128)
+    torch.cuda.synchronize()
+    assert torch.equal(got, want)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        got = prefill_attention(q, k, v, plan, 0.1, 128)
+    for _ in range(2):
+        got.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(got, want)
