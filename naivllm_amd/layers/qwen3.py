@@ -291,42 +291,32 @@ def lm_head_rows(hidden: int) -> int:
     return max(16, min(79, LM_HEAD_LDS // ((hidden + 8) * 2)))
 
 
-def prefill_metadata(token_lists, starts, tables, block_size: int, q_block: int, device):
-    """Rows of one prefill forward over several sequences' new tokens.
-
-    Sequence i contributes its tokens starts[i] .. len(token_lists[i]) - 1 at
-    their positions (the pages before starts[i] already hold their KV: a
-    cached prefix).  Its rows are cut into causal blocks of q_block rows;
-    each block is one entry of the verify attention's batch, whose context
-    ends at the block's last position and whose block-table row is the
-    sequence's, so every row attends exactly the keys 0 .. its position.
-    Returns (input_ids, positions, slot_mapping, block_tables, context_lens,
-    cu_seqlens_q, last_rows) on ``device``; last_rows[i] is the row of
-    sequence i's last token."""
+def prefill_rows(token_lists, starts, tables, block_size: int):
+    """Rows of one prefill forward over several sequences' new tokens, as
+    numpy arrays: sequence i contributes its tokens starts[i] ..
+    len(token_lists[i]) - 1 at their positions (the pages before starts[i]
+    already hold their KV: a cached prefix).
+    Returns (input_ids, positions, slot_mapping, last_rows, block_tables, new,
+    lens): last_rows[i] is the row of sequence i's last token, block_tables
+    has one row per sequence (-1 padded), and new / lens are the sequences'
+    new and whole lengths."""
     import numpy as np
 
-    ids, pos, slots, ctx, cu, bt_rows, last = [], [], [], [], [0], [], []
-    width = max(len(t) for t in tables)
-    for toks, start, table in zip(token_lists, starts, tables):
-        n = len(toks)
+    if not len(token_lists) == len(starts) == len(tables):
+        raise ValueError(f"{len(token_lists)} token lists, {len(starts)} starts and {len(tables)} block tables")
+    lens = [len(t) for t in token_lists]
+    for n, start in zip(lens, starts):
         if not 0 <= start < n:
             raise ValueError(f"prefill start {start} outside a {n}-token sequence")
-        p = np.arange(start, n, dtype=np.int64)
-        page = np.asarray(table, dtype=np.int64)[p // block_size]
-        ids.append(np.asarray(toks[start:], dtype=np.int64))
-        pos.append(p)
-        slots.append(page * block_size + p % block_size)
-        row = np.full(width, -1, dtype=np.int32)
-        row[:len(table)] = table
-        for b0 in range(start, n, q_block):
-            b1 = min(n, b0 + q_block)
-            ctx.append(b1)
-            cu.append(cu[-1] + (b1 - b0))
-            bt_rows.append(row)
-        last.append(cu[-1] - 1)
-    t = lambda x, dt: torch.from_numpy(np.ascontiguousarray(x, dtype=dt)).to(device)  # noqa: E731
-    return (t(np.concatenate(ids), np.int64), t(np.concatenate(pos), np.int64), t(np.concatenate(slots), np.int64),
-            t(np.stack(bt_rows), np.int32), t(ctx, np.int64), t(cu, np.int32), t(last, np.int64))
+    new = [n - start for n, start in zip(lens, starts)]
+    pos = [np.arange(start, n, dtype=np.int64) for n, start in zip(lens, starts)]
+    slots = [np.asarray(t, dtype=np.int64)[p // block_size] * block_size + p % block_size for t, p in zip(tables, pos)]
+    ids = [np.asarray(t[start:], dtype=np.int64) for t, start in zip(token_lists, starts)]
+    bt = np.full((len(tables), max(len(t) for t in tables)), -1, dtype=np.int32)
+    for row, t in zip(bt, tables):
+        row[:len(t)] = t
+    last = np.cumsum(new, dtype=np.int64) - 1
+    return np.concatenate(ids), np.concatenate(pos), np.concatenate(slots), last, bt, new, lens
 
 
 def fused_rows(hidden_size: int) -> int:
@@ -391,11 +381,6 @@ class Qwen3Verify:
             _lib.check(_lib.lib().nsv_lm_head_pack(self.lm_head.data_ptr(), self.lm_head_packed.data_ptr(), V, E,
                                                    _lib.stream_ptr(self.device)), "lm_head_pack")
 
-    def prefill_q_block(self) -> int:
-        """Query rows per causal block of a prefill: the verify kernel serves
-        up to 64 (GQA group x rows) per (sequence, kv head)."""
-        return 64 // (self.cfg.num_heads // self.cfg.num_kv_heads)
-
     def _wide_splits(self, T: int) -> tuple[int, int, int] | None:
         """Splits of the qkv, o and down projections where T rows run on the
         weight-streaming kernel, else None."""
@@ -415,19 +400,9 @@ class Qwen3Verify:
         last token come back, [len(token_lists), vocab]."""
         import numpy as np
 
-        bs, lens = self.block_size, [len(t) for t in token_lists]
-        for n, start in zip(lens, starts):
-            if not 0 <= start < n:
-                raise ValueError(f"prefill start {start} outside a {n}-token sequence")
-        new = [n - start for n, start in zip(lens, starts)]
-        pos = [np.arange(start, n, dtype=np.int64) for n, start in zip(lens, starts)]
-        slots = [np.asarray(t, dtype=np.int64)[p // bs] * bs + p % bs for t, p in zip(tables, pos)]
-        ids = [np.asarray(t[start:], dtype=np.int64) for t, start in zip(token_lists, starts)]
-        bt = np.full((len(tables), max(len(t) for t in tables)), -1, dtype=np.int32)
-        for row, t in zip(bt, tables):
-            row[:len(t)] = t
-        last = np.cumsum(new, dtype=np.int64) - 1
-        rows = _lib.upload(np.concatenate([*ids, *pos, *slots, last]), self.device)
+        bs = self.block_size
+        *per_row, last, bt, new, lens = prefill_rows(token_lists, starts, tables, bs)
+        rows = _lib.upload(np.concatenate([*per_row, last]), self.device)
         T = sum(new)
         plan = PrefillPlan(new, lens, self.cfg.num_heads, self.cfg.num_kv_heads, bs, self.device)
         return self.forward(rows[:T], rows[T:2 * T], rows[2 * T:3 * T], _lib.upload(bt, self.device), None, None, 0,

@@ -141,7 +141,7 @@ class DraftRunner:
     def prefill(self, seqs, starts=None) -> None:
         """KV of the tokens of each sequence from ``starts[i]`` (default 0: the
         draft pool's own prefix is empty) in one forward over every sequence
-        (Qwen3Verify.prefill: causal blocks through the verify kernel)."""
+        (Qwen3Verify.prefill)."""
         if not seqs:
             return
         starts = [0] * len(seqs) if starts is None else list(starts)
