@@ -61,7 +61,7 @@ constexpr int wl_max(int a, int b) { return a > b ? a : b; }
 // EPI 0: plain; 1: SwiGLU.  NW waves: NW / WK column slots, WK waves sharing
 // each slot's reduction.
 template <int MT, int EPI, int NW, int WK, int NTW, bool PACKED>
-__global__ __launch_bounds__(NW * 64, NW > 8 ? 3 : 2) void wide_linear_kernel(WideArgs a) {
+__global__ __launch_bounds__(NW * 64, 2) void wide_linear_kernel(WideArgs a) {
   constexpr int NT = NW * 64, WN = NW / WK;
   constexpr int MP = MT * 16;
   constexpr int Q = 4 / WK;                       // 64-element groups per wave and chunk
@@ -323,13 +323,15 @@ struct WidePlan {
 // of two waves do not hold (108 rows: 54.7 against 74.4).
 WidePlan wide_plan(int M, int N, int K, int epi, bool packed, int cus) {
   if (M <= 0 || M > kWlMaxRows || N <= 0 || K <= 0 || N % 16 || K % kWlKC) return {0, 0};
-  if ((int64_t)N * K * 2 > ((int64_t)1 << 31) - (1 << 20)) return {0, 0};  // byte offsets fit an int
+  // byte offsets into the weight and into the activations' padded row tiles fit an int
+  const int64_t rows = (M + 15) / 16 * 16 < 32 ? 32 : (M + 15) / 16 * 16;
+  if ((N > rows ? N : rows) * (int64_t)K * 2 > ((int64_t)1 << 31) - (1 << 20)) return {0, 0};
   if (epi == 1) {
     if (N % 32 || packed) return {0, 0};
     if (N / 32 <= cus) return {16, 1};
     return {M <= 80 ? 48 : 64, 1};
   }
-  if (packed) return {128, 1};
+  if (packed) return {128, K == 1024 || K == 2048 || K == 4096 ? 1 : 0};  // the packed layout's reductions
   const int nck = K / kWlKC;
   auto even = [&](int cols) {
     const int groups = (N + cols - 1) / cols;

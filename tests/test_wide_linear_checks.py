@@ -61,3 +61,19 @@ def test_sum_consumers_check_their_rows():
     with pytest.raises(ValueError, match="slot_mapping"):
         qm.qk_norm_rope_store_sum(part, 2, z(128), z(128), z(M, 128, dtype=F32), z(M - 1, dtype=torch.int64),
                                   z(M, 4, 128), z(2, 16, 2, 128), z(2, 16, 2, 128), 4, 2, 128, 1e-6)
+
+
+@pytest.mark.parametrize("M,N,K,taken", [
+    (128, 16, 1 << 25, False),  # 2^30 bytes of weight, 2^33 of activations
+    (128, 16, 1 << 23, False),  # 2^31 of activations, the first past an int
+    (128, 16, (1 << 23) - (1 << 13), True),
+    (1, 16, 1 << 25, False),    # one row is padded to two row tiles
+    (128, 1 << 18, 4096, False),  # 2^31 of weight
+    (128, 151936, 4096, True),
+])
+def test_shapes_past_32_bit_offsets_are_not_taken(M, N, K, taken):
+    assert (qm.wide_splits(M, N, K) > 0) == taken
+
+
+def test_packed_takes_the_packed_layouts_reductions():
+    assert [qm.wide_splits(80, 1024, K, packed=True) for K in (512, 1024, 2048, 3072, 4096, 5120)] == [0, 1, 1, 0, 1, 0]
