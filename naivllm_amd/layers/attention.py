@@ -251,6 +251,14 @@ class PrefillPlan:
         self.work.record_stream(stream)
 
 
+def _aligned(t: torch.Tensor) -> torch.Tensor:
+    """A contiguous tensor whose data starts on 16 bytes, as the loads of the
+    prefill kernel that go straight to LDS need it (a view at an odd offset is
+    copied; what torch allocates is aligned)."""
+    t = t.contiguous()
+    return t if t.data_ptr() % 16 == 0 else t.clone()
+
+
 def prefill_attention(query: torch.Tensor, k: torch.Tensor, v: torch.Tensor, plan: PrefillPlan, scale: float,
                       head_dim: int, block_tables: torch.Tensor | None = None) -> torch.Tensor:
     """Causal attention of a prefill step's rows (bf16): query [rows, H, D];
@@ -267,7 +275,6 @@ def prefill_attention(query: torch.Tensor, k: torch.Tensor, v: torch.Tensor, pla
     if block_tables is None:
         if tuple(k.shape) != tuple(v.shape) or tuple(k.shape[1:]) != (Hkv, head_dim) or k.shape[0] < plan.keys:
             raise ValueError(f"k and v must be (at least {plan.keys}, {Hkv}, {head_dim}), got {tuple(k.shape)}")
-        k, v = k.contiguous(), v.contiguous()
     else:
         nb, bs, hkv, d = _check_cache(k, "k_cache")
         if tuple(v.shape) != (nb, bs, hkv, d) or not v.is_contiguous():
@@ -278,7 +285,7 @@ def prefill_attention(query: torch.Tensor, k: torch.Tensor, v: torch.Tensor, pla
         if block_tables.shape[0] < plan.sequences:
             raise ValueError(f"{plan.sequences} sequences but {block_tables.shape[0]} block-table rows")
         max_blocks = block_tables.shape[1]
-    query = query.contiguous()
+    query, k, v = _aligned(query), _aligned(k), _aligned(v)
     out = torch.empty_like(query)
     # (the plan's list is the only memory that calls on several streams or
     # threads share, and they only read it)

@@ -386,8 +386,10 @@ class Qwen3Verify:
         weight-streaming kernel, else None."""
         cfg = self.cfg
         E, I, HD = cfg.hidden_size, cfg.intermediate_size, cfg.num_heads * cfg.head_dim
+        # (its loads take weights on 16 bytes: a view at an odd offset stays on hipBLASLt)
         if T > WIDE_ROWS or E % 4 or E > 4096 or not all(
-                L[k].is_contiguous() for L in self.layers for k in ("qkv", "o", "gate_up", "down")):
+                L[k].is_contiguous() and L[k].data_ptr() % 16 == 0
+                for L in self.layers for k in ("qkv", "o", "gate_up", "down")):
             return None
         n = (wide_splits(T, HD + 2 * cfg.num_kv_heads * cfg.head_dim, E), wide_splits(T, E, HD), wide_splits(T, E, I))
         return n if min(*n, wide_splits(T, 2 * I, E, swiglu=True)) > 0 else None

@@ -94,3 +94,20 @@ def test_a_plan_serves_other_streams_and_captures():
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(got, want)
+
+
+def test_rows_at_odd_offsets():
+    # contiguous views that start 2 bytes into an allocation give the aligned rows' output
+    print("case: prefill attention from views at odd offsets", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(4)
+    base = torch.randn(3, 150 * 2 * 128 + 1, generator=g, device="cuda").bfloat16()
+    q, k, v = (b[1:].view(150, -1, 128)[:, :n].contiguous() for b, n in zip(base, (2, 1, 1)))
+    plan = PrefillPlan([150], [150], 2, 1, None, q.device)
+    want = prefill_attention(q, k, v, plan, 0.1, 128)
+    odd = []
+    for t in (q, k, v):
+        flat = torch.empty(t.numel() + 1, dtype=t.dtype, device="cuda")
+        flat[1:].copy_(t.reshape(-1))
+        odd.append(flat[1:].view(t.shape))
+        assert odd[-1].data_ptr() % 16 == 2
+    assert torch.equal(prefill_attention(*odd, plan, 0.1, 128), want)

@@ -68,3 +68,13 @@ def test_a_capture_holds_no_outside_event(streams):
     streams[1][0] = True
     plan.use_on(other)
     assert other.waits == [] and plan.work.uses == []
+
+
+def test_views_at_odd_offsets_are_copied():
+    base = torch.arange(4 * 2 * 64 + 8, dtype=torch.bfloat16)
+    for off in (0, 8):  # whole 16 bytes
+        t = base[off:off + 512].view(4, 2, 64)
+        assert at._aligned(t) is t
+    for off in (1, 4):
+        t = base[off:off + 512].view(4, 2, 64)
+        assert t.is_contiguous() and at._aligned(t).data_ptr() % 16 == 0 and torch.equal(at._aligned(t), t)
