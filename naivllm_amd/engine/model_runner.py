@@ -163,6 +163,9 @@ class ModelRunner:
         width = v["block_tables"].shape[1]
         if any(len(self._table(s)) > width for s in seqs):
             raise ValueError("block table longer than the runner's max_model_length allows")
+        if self._inputs.is_cuda and torch.cuda.is_current_stream_capturing():
+            # (a replay would read a host copy that later calls have overwritten)
+            raise RuntimeError("run_spec_verify reads host sequences: it cannot be captured in a graph")
         i, self._next = self._next, (self._next + 1) % STAGING
         if self._copied[i] is not None:
             self._copied[i].synchronize()

@@ -115,3 +115,20 @@ def test_calls_in_a_row_keep_their_own_inputs():
     torch.cuda.synchronize()
     for i, g in enumerate(got):
         assert torch.equal(g, want[i % 3]), i
+
+
+def test_a_call_inside_a_capture_is_refused():
+    # its inputs are host values; refused before any staging copy is taken
+    model, seqs = setup(9)
+    runner = ModelRunner(model, max_num_sequences=4, num_spec_tokens=K, max_model_length=256)
+    want = runner.run_spec_verify(seqs).clone()
+    torch.cuda.synchronize()
+    x = torch.zeros(4, device="cuda")
+    graph = torch.cuda.CUDAGraph()
+    before = runner._next
+    with torch.cuda.graph(graph):
+        x.add_(1)
+        with pytest.raises(RuntimeError, match="captured"):
+            runner.run_spec_verify(seqs)
+    assert runner._next == before
+    assert torch.equal(runner.run_spec_verify(seqs), want)
