@@ -76,6 +76,9 @@ constexpr float kNegInf = -__builtin_inff();
 // how far (log2 domain) a row's running maximum may pass its exponent reference
 // before the key-split kernel moves the reference (weights stay <= 2^8)
 constexpr float kRefSlack = 8.f;
+// how far (log2 domain) a row's running sum may lie above a tile's maximum for
+// the reference to move down to that maximum (fine references, below)
+constexpr float kRefDropSum = 65536.f;
 
 // Timeline stamps (a build knob: libnaivspec_stamp.so is built with
 // NSV_STAMP=1; the default library has no stamp code).  Thread 0 of every
@@ -212,13 +215,20 @@ __device__ __forceinline__ int num_splits(const VerifyArgs& a, int ctx) {
 // 10.2, 9,000 24.6 -> 21.3; 64 pairs (4 splits) 100 keys 8.4 -> 6.8; two
 // splits at 300 keys instead of one 9.0; 4 rows, one tile, 300 keys: one
 // split 7.0 against 6.8 for eight.
+//
+// fine: the context takes fewer splits than the plan's, so a wave takes more
+// tiles; its exponent reference then follows every tile's maximum (see the
+// kernel), or its heavy weights would be rounded to bf16 where the plan's
+// splits, with about one tile per wave, hold them exactly.
 template <int MT>
-__device__ __forceinline__ int split_len_ks(const VerifyArgs& a, int ctx) {
+__device__ __forceinline__ int split_len_ks(const VerifyArgs& a, int ctx, bool& fine) {
+  fine = false;
   if (a.split_tokens > 0) return a.split_tokens;
   int n = a.ks_splits;
   if (n > 8) n = max(8, min(n, ctx >> 9));
   if (MT > 1 && ctx <= 512) n = min(n, 4);
   if (ctx <= (MT > 1 ? 320 : 200)) n = 1;
+  fine = n < a.ks_splits;
   const int per = div_small(ctx + n - 1, n);
   return per <= 16 ? 16 : (per + 15) & ~15;
 }
@@ -1024,7 +1034,8 @@ __global__ __launch_bounds__(NW * 64, 8 / NW) void verify_attn_ks_kernel(VerifyA
   if (pair_raw >= a.npairs) return;
   const int ctx = clamp_context(a, ctx_raw);
   const int qlen = q1 - q0;
-  const int len = split_len_ks<MT>(a, ctx);
+  bool fine;
+  const int len = split_len_ks<MT>(a, ctx, fine);
   const int nsplit = num_splits_ks(ctx, len);
   if (split >= nsplit || qlen < 0) return;  // uniform per workgroup
   const int kb = split * len;
@@ -1209,6 +1220,15 @@ __global__ __launch_bounds__(NW * 64, 8 / NW) void verify_attn_ks_kernel(VerifyA
     // accumulators are still zero then).  The weights are a constant factor
     // times the ones a reference at the running maximum would give, and their
     // bf16 rounding is relative, so the result is the same softmax.
+    //
+    // A weight at its reference is exactly 1 in bf16, so the error falls with
+    // the number of references a row has.  With fine (uniform) the reference
+    // is every tile's own maximum, moved down too while the running sum stays
+    // within kRefDropSum of it (a weight stays <= 1 then).  8 pairs, N(0, 1)
+    // scores, error against 64 bits in 1e-5 (plan's splits; these splits with
+    // a lazy reference -> fine): 300 keys, 18 rows 194; 218 -> 194, 150 keys
+    // 195; 201 -> 195, 4,000 keys of a 130-page table 194; 225 -> 194; time per
+    // call 8.4 -> 7.9 us (300 keys), 10.5 -> 10.1 (1,250), 14.8 -> 14.1 (4,000).
     i16x4 pB[MT];
     float alpha[MT];
     bool moved = false;
@@ -1217,11 +1237,14 @@ __global__ __launch_bounds__(NW * 64, 8 / NW) void verify_attn_ks_kernel(VerifyA
       float mx = __builtin_fmaxf(__builtin_fmaxf(sacc[mt][0], sacc[mt][1]), __builtin_fmaxf(sacc[mt][2], sacc[mt][3]));
       mx = row_max4(mx);
       const float m_old = m_run[mt];
-      const float m_new = fmaxf(m_old, mx);
-      // (m_old -inf and m_new finite: +inf, a move; both -inf: NaN, none)
-      const bool shift = (m_new - m_old) * sc > kRefSlack;
+      const float m_new = fine ? mx : fmaxf(m_old, mx);
+      const float al = __builtin_amdgcn_exp2f((m_old - m_new) * sc);
+      // (m_old -inf and m_new finite: +inf, a move; both -inf: NaN, none; fine
+      // and no key for a row, m_new -inf: none)
+      const bool shift = fine ? mx > m_old || (mx > kNegInf && l_run[mt] * al <= kRefDropSum)
+                              : (m_new - m_old) * sc > kRefSlack;
       const float m_ref = shift ? m_new : m_old;
-      alpha[mt] = shift ? __builtin_amdgcn_exp2f((m_old - m_new) * sc) : 1.f;
+      alpha[mt] = shift ? al : 1.f;
       moved |= shift && m_old != kNegInf;
       const float nb = (m_ref == kNegInf) ? 0.f : -m_ref * sc;  // exp2 bias
       float p[4];

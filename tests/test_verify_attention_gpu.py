@@ -269,3 +269,33 @@ def test_split_counts_follow_the_context(G, ql):
     assert _kernel(vb, ql) == "key-split"
     out = _gpu(vb, max_q_len=ql)
     assert_close(out, _oracle(vb), "bf16", "splits by context")
+
+
+@pytest.mark.parametrize("rows,ctx", [(9, 300), (2, 150), (9, 1250), (9, 4000)])
+def test_fewer_splits_are_no_less_precise(rows, ctx):
+    # a table much wider than the context: the splits are counted by the
+    # context, and the error against 64 bits stays that of splits whose waves
+    # take one 16-key tile each (every tile its own exponent reference).  The
+    # same references give the same rounding up to the splits' merge order, a
+    # few permille; one reference per wave gives 3 to 15 percent more.
+    print(f"case: verify attention precision rows={rows} ctx={ctx}", flush=True)
+    H, Hkv, D, page, width = 16, 8, 128, 64, 520
+    g = torch.Generator(device="cuda").manual_seed(ctx + rows)
+    rand = lambda *s: torch.randn(*s, generator=g, device="cuda").bfloat16()  # noqa: E731
+    B, npg = 1, -(-ctx // page)  # 8 pairs: the plan takes 32 splits of such a table
+    q, k, v = rand(B * rows, H, D), rand(B * npg, page, Hkv, D), rand(B * npg, page, Hkv, D)
+    bt = torch.full((B, width), -1, dtype=torch.int32)
+    bt[:, :npg] = torch.arange(B * npg, dtype=torch.int32).view(B, npg)
+    lens = torch.full((B,), ctx, dtype=torch.int64, device="cuda")
+    cu = torch.arange(0, B * rows + 1, rows, dtype=torch.int32, device="cuda")
+    pos = torch.arange(ctx - rows, ctx, device="cuda").repeat(B)
+    run = lambda split: paged_attention_verify(  # noqa: E731
+        q, k, v, bt.cuda(), lens, cu, pos, D ** -0.5, H, Hkv, D, page, 16, max_q_len=rows, kv_split_tokens=split).double()
+    kd, vd = (t.double().view(B, npg * page, Hkv, D)[:, :ctx].permute(0, 2, 1, 3).repeat_interleave(H // Hkv, 1)
+              for t in (k, v))
+    s = torch.matmul(q.double().view(B, rows, H, D).permute(0, 2, 1, 3), kd.transpose(2, 3).contiguous()) * D ** -0.5
+    s.masked_fill_(torch.arange(ctx, device="cuda")[None] > pos[:rows, None], -float("inf"))
+    want = torch.matmul(s.softmax(-1), vd.contiguous()).permute(0, 2, 1, 3).reshape(B * rows, H, D)
+    assert verify_attention_plan(B, H, Hkv, D, page, width, rows, torch.bfloat16)[0] == "key-split"
+    err = [((run(split) - want).norm() / want.norm()).item() for split in (0, 128)]
+    assert err[0] <= 1.01 * err[1], err
