@@ -114,7 +114,7 @@ def test_qk_norm_rope_store_of_a_sum(splits):
 def test_head_writes_or_refuses_the_callers_logits():
     # 96 rows at hidden 1024: past the streaming head's rows, on the packed copy
     print("case: logits_out of the wide head", flush=True)
-    cfg = qm.Qwen3Config(vocab_size=65536, hidden_size=1024, num_layers=1, num_heads=4, num_kv_heads=2, head_dim=64,
+    cfg = qm.Qwen3Config(vocab_size=131072, hidden_size=1024, num_layers=1, num_heads=4, num_kv_heads=2, head_dim=64,
                          intermediate_size=512, max_position=256)
     model = qm.Qwen3Verify(cfg, "cuda", seed=3)
     model.allocate_kv_cache(8, 16)
