@@ -47,9 +47,12 @@ constexpr int kWaveRows = 32;      // query rows per wave
 constexpr int kMaxPages = 2048;    // block-table entries staged in LDS
 constexpr int kTileWords = 8;      // int32 words of a tile record
 constexpr float kNegInf = -__builtin_inff();
-// how far (log2 domain) a row's maximum may pass its exponent reference
-// before the reference moves (weights stay <= 2^8, far inside fp32)
-constexpr float kRefSlack = 8.f;
+// keys of a workgroup's range up to which every 32 keys have an exponent
+// reference of their own, every 64 beyond
+constexpr int kFineKeys = 256;
+// how far (log2 domain) a maximum may lie below the row's running one for the
+// reference to move down to it (sums stay within 2^16 of their count)
+constexpr float kRefDrop = 16.f;
 
 struct PrefillArgs {
   const bf16_t* q;
@@ -209,7 +212,7 @@ __global__ __launch_bounds__(NW * 64, 2) void prefill_attn_kernel(PrefillArgs a)
   for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
     for (int i = 0; i < 16; ++i) acc[dt][i] = 0.f;
-  float m_ref = kNegInf, l_run = 0.f;
+  float m_ref = kNegInf, m_run = kNegInf, l_run = 0.f;  // exponent reference, running maximum, running sum
   const float sc = a.scale_log2;
 
   f32x16 s[2];
@@ -268,24 +271,46 @@ __global__ __launch_bounds__(NW * 64, 2) void prefill_attn_kernel(PrefillArgs a)
         for (int i = 0; i < 16; ++i)
           s[t][i] = (mapped >> (t * 32 + (i >> 2) * 8 + (i & 3))) & 1 ? s[t][i] : kNegInf;
     }
-    float mx = fmaxf(s[0][0], s[1][0]);
+    // A weight at its exponent reference is exactly 1 in bf16, every other is
+    // rounded: the error falls with the number of references a row has, so
+    // the reference is the maximum of each group of 32 keys at first and of
+    // each tile later, moved down as well as up (a weight stays <= 1, and the
+    // sums within 2^kRefDrop of their count).  Error against 64 bits at N(0, 1)
+    // scores, in 1e-5 (the verify kernel on causal blocks; one reference,
+    // moved lazily -> these): one prompt of 1,206 tokens 193; 204 -> 192, 40
+    // rows behind 256 keys 203; 229 -> 203, 900 behind 2,048 216; 231 -> 205.
+    // The rescaling costs up to 14% of the time (2,900 and 4,050 rows of 32/8
+    // heads behind 4,096 keys 721 -> 822 us, 8,192 tokens 538 -> 600, one
+    // prompt of 1,206 33 -> 34).  A reference every 64 keys from the first key
+    // on takes 33 us there, but is 1 to 3% further off than the verify kernel
+    // (1,206 tokens 196, 40 rows behind 256 keys 209).
+    const bool fine = n0 < key_begin + kFineKeys;  // uniform
+    float mx[2];
 #pragma unroll
-    for (int i = 1; i < 16; ++i) mx = fmaxf(fmaxf(mx, s[0][i]), s[1][i]);
-    mx = half_max(mx);
-    // the exponent reference follows the running maximum only when it is
-    // passed by more than 2^kRefSlack (always on a row's first key)
-    const bool move = mx > kNegInf && !((mx - m_ref) * sc <= kRefSlack);
-    if (__ballot(move)) {
-      const float mn = move ? mx : m_ref;
-      const float alpha = !move ? 1.f : m_ref == kNegInf ? 0.f : __builtin_amdgcn_exp2f((m_ref - mn) * sc);
+    for (int t = 0; t < 2; ++t) {
+      mx[t] = s[t][0];
+#pragma unroll
+      for (int i = 1; i < 16; ++i) mx[t] = fmaxf(mx[t], s[t][i]);
+    }
+    mx[0] = half_max(fine ? mx[0] : fmaxf(mx[0], mx[1]));
+    // the reference moved to a group's maximum; returns the factor of what was summed before
+    auto move = [&](float m) {
+      m_run = fmaxf(m_run, m);
+      const bool on = m > kNegInf && !((m_run - m) * sc > kRefDrop);
+      const float alpha = on ? __builtin_amdgcn_exp2f((m_ref - m) * sc) : 1.f;  // (from -inf: 0)
+      m_ref = on ? m : m_ref;
       l_run *= alpha;
+      return alpha;
+    };
+    auto rescale = [&](float alpha) {
+      if (!__ballot(alpha != 1.f)) return;
 #pragma unroll
       for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
         for (int i = 0; i < 16; ++i) acc[dt][i] *= alpha;
-      m_ref = mn;
-    }
-    const float nb = m_ref == kNegInf ? 0.f : -m_ref * sc;
+    };
+    rescale(move(mx[0]));
+    float nb = m_ref == kNegInf ? 0.f : -m_ref * sc;
     // O^T += V^T P^T, 16 keys per step: element j of lane half h is key
     // 8 (j / 4) + 4 h + j % 4 of the step in both operands.  A step's weights
     // are computed, and its V operands read, during the step before's products.
@@ -321,8 +346,14 @@ __global__ __launch_bounds__(NW * 64, 2) void prefill_attn_kernel(PrefillArgs a)
     weights(0);
 #pragma unroll
     for (int st = 0; st < ST; ++st) {
+      const bool second = fine && st + 1 == ST / 2;  // the second 32 keys come next
+      float alpha = 1.f;
       if (st + 1 < ST) {
         read(st + 1);
+        if (second) {  // uniform
+          alpha = move(half_max(mx[1]));
+          nb = m_ref == kNegInf ? 0.f : -m_ref * sc;
+        }
         weights(st + 1);
       }
 #pragma unroll
@@ -330,6 +361,7 @@ __global__ __launch_bounds__(NW * 64, 2) void prefill_attn_kernel(PrefillArgs a)
         const uint2 lo = va[st & 1][dt][0], hi = va[st & 1][dt][1];
         acc[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_bf16x8(u32x4{lo.x, lo.y, hi.x, hi.y}), pB[st & 1], acc[dt], 0, 0, 0);
       }
+      if (second) rescale(alpha);
       __builtin_amdgcn_sched_barrier(0);
     }
   };

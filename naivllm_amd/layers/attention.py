@@ -233,10 +233,11 @@ class PrefillPlan:
         self.num_heads, self.num_kv_heads, self.block_size = num_heads, num_kv_heads, block_size
         self.sequences, self.rows, self.keys = len(seqlens_q), int(sum(seqlens_q)), int(sum(seqlens_k))
         self.work = work.to(device, non_blocking=ahead)
-        self.stream = torch.cuda.current_stream(device)
+        stream = torch.cuda.current_stream(device)
+        self.stream = stream.cuda_stream
         self.ready = torch.cuda.Event() if ahead else None  # the transfer is done
         if ahead:
-            self.ready.record(self.stream)
+            self.ready.record(stream)
 
     def use_on(self, stream) -> None:
         """Order work enqueued on ``stream`` after the transfer, and keep the
@@ -244,7 +245,7 @@ class PrefillPlan:
         can hold no wait for an event from outside it, and needs none:
         torch.cuda.graph waits for the device before it begins, and whoever
         replays the graph keeps the plan."""
-        if stream == self.stream or torch.cuda.is_current_stream_capturing():
+        if stream.cuda_stream == self.stream or torch.cuda.is_current_stream_capturing():
             return
         if self.ready is not None:
             stream.wait_event(self.ready)
@@ -252,10 +253,9 @@ class PrefillPlan:
 
 
 def _aligned(t: torch.Tensor) -> torch.Tensor:
-    """A contiguous tensor whose data starts on 16 bytes, as the loads of the
-    prefill kernel that go straight to LDS need it (a view at an odd offset is
-    copied; what torch allocates is aligned)."""
-    t = t.contiguous()
+    """t on 16 bytes, as the loads of the prefill kernel that go straight to
+    LDS need it: a view at an odd offset is copied (what torch allocates is
+    aligned)."""
     return t if t.data_ptr() % 16 == 0 else t.clone()
 
 
@@ -275,6 +275,7 @@ def prefill_attention(query: torch.Tensor, k: torch.Tensor, v: torch.Tensor, pla
     if block_tables is None:
         if tuple(k.shape) != tuple(v.shape) or tuple(k.shape[1:]) != (Hkv, head_dim) or k.shape[0] < plan.keys:
             raise ValueError(f"k and v must be (at least {plan.keys}, {Hkv}, {head_dim}), got {tuple(k.shape)}")
+        k, v = k.contiguous(), v.contiguous()
     else:
         nb, bs, hkv, d = _check_cache(k, "k_cache")
         if tuple(v.shape) != (nb, bs, hkv, d) or not v.is_contiguous():
@@ -285,18 +286,21 @@ def prefill_attention(query: torch.Tensor, k: torch.Tensor, v: torch.Tensor, pla
         if block_tables.shape[0] < plan.sequences:
             raise ValueError(f"{plan.sequences} sequences but {block_tables.shape[0]} block-table rows")
         max_blocks = block_tables.shape[1]
-    query, k, v = _aligned(query), _aligned(k), _aligned(v)
+    query = query.contiguous()
+    if (query.data_ptr() | k.data_ptr() | v.data_ptr()) % 16:
+        query, k, v = _aligned(query), _aligned(k), _aligned(v)
     out = torch.empty_like(query)
     # (the plan's list is the only memory that calls on several streams or
     # threads share, and they only read it)
-    plan.use_on(torch.cuda.current_stream(query.device))
+    stream = torch.cuda.current_stream(query.device)
+    plan.use_on(stream)
     part = torch.empty(plan.slots * H * plan.tile_rows * (head_dim + 2), dtype=torch.float32,
                        device=query.device) if plan.slots else None
     tiles = plan.work.data_ptr()
     rc = _lib.lib().nsv_prefill_attention(
         out.data_ptr(), query.data_ptr(), k.data_ptr(), v.data_ptr(), _lib.ptr(block_tables), tiles, plan.ntiles,
         plan.tile_rows, tiles + plan.ntiles * 32, plan.nmerges, float(scale), H, Hkv, head_dim,
-        plan.block_size or 1, max_blocks, _lib.ptr(part), _lib.stream_ptr(query.device))
+        plan.block_size or 1, max_blocks, _lib.ptr(part), stream.cuda_stream)
     _lib.check(rc, "prefill_attention")
     return out
 

@@ -8,7 +8,7 @@ import pytest
 import torch
 
 from gpu_util import assert_close
-from naivllm_amd.layers.attention import PrefillPlan, prefill_attention, prefill_tiles
+from naivllm_amd.layers.attention import PrefillPlan, paged_attention_verify, prefill_attention, prefill_tiles
 from naivllm_amd.utils import synth
 from oracle import attention as ora
 
@@ -111,3 +111,33 @@ def test_rows_at_odd_offsets():
         odd.append(flat[1:].view(t.shape))
         assert odd[-1].data_ptr() % 16 == 2
     assert torch.equal(prefill_attention(*odd, plan, 0.1, 128), want)
+
+
+@pytest.mark.parametrize("new,keys", [(40, 296), (270, 526), (300, 1324), (1000, 1000)])
+def test_prefill_is_no_less_precise_than_verify(new, keys):
+    # error against 64 bits beside that of the verify kernel over causal blocks
+    # of 64 / G rows: both round each weight to bf16 once, and a weight at its
+    # exponent reference not at all, so the kernel with fewer references per
+    # row is further off (one lazily moved reference: 5 to 12 percent); a
+    # permille is the spread of equal counts
+    print(f"case: prefill precision, {new} rows of {keys} keys", flush=True)
+    H, Hkv, D, page = 16, 8, 128, 64
+    g = torch.Generator(device="cuda").manual_seed(keys)
+    rand = lambda *s: torch.randn(*s, generator=g, device="cuda").bfloat16()  # noqa: E731
+    npg, block = -(-keys // page), 64 // (H // Hkv)
+    q, k, v = rand(new, H, D), rand(npg, page, Hkv, D), rand(npg, page, Hkv, D)
+    bt = torch.arange(npg, dtype=torch.int32, device="cuda")[None]
+    first = list(range(keys - new, keys, block))
+    ends = [min(keys, b + block) for b in first]
+    pos = torch.arange(keys - new, keys, device="cuda")
+    blocks = paged_attention_verify(
+        q, k, v, bt.repeat(len(ends), 1), torch.tensor(ends, device="cuda"),
+        torch.tensor([0] + [e - keys + new for e in ends], dtype=torch.int32, device="cuda"), pos, D ** -0.5, H, Hkv, D,
+        page, block, max_q_len=block)
+    got = prefill_attention(q, k, v, PrefillPlan([new], [keys], H, Hkv, page, q.device), D ** -0.5, D, bt)
+    kd, vd = (t.double().view(npg * page, Hkv, D)[:keys].permute(1, 0, 2).repeat_interleave(H // Hkv, 0) for t in (k, v))
+    s = torch.matmul(q.double().permute(1, 0, 2), kd.transpose(1, 2).contiguous()) * D ** -0.5
+    s.masked_fill_(torch.arange(keys, device="cuda")[None] > pos[:, None], -float("inf"))
+    want = torch.matmul(s.softmax(-1), vd.contiguous()).permute(1, 0, 2)
+    err = [((x.double() - want).norm() / want.norm()).item() for x in (got, blocks)]
+    assert err[0] <= 1.005 * err[1], err

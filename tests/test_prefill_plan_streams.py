@@ -10,7 +10,7 @@ import naivllm_amd.layers.attention as at
 
 class Stream:
     def __init__(self, name):
-        self.name, self.waits = name, []
+        self.cuda_stream, self.waits = name, []
 
     def wait_event(self, event):
         self.waits.append(event)
