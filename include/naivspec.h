@@ -110,8 +110,7 @@ int nsv_verify_attention(void* out, const void* q, const void* k_cache,
  *   tiles   [ntiles, 8], merges [nmerges, 4] int32, device memory; heavier
  *           tiles first fill the chip best
  * Supported: D in {64, 128}; H % Hkv == 0; tile_rows 64 or 128 when H / Hkv
- * is even, 128 or 256 otherwise; block_size a power of two, a record's keys
- * on at most 2048 pages.
+ * is even, 128 or 256 otherwise; block_size a power of two.
  */
 int nsv_prefill_attention(void* out, const void* q, const void* k,
                           const void* v, const int32_t* block_tables,

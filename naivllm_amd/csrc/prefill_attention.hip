@@ -44,7 +44,7 @@ typedef __attribute__((address_space(3))) i16x4 lds_i16x4;
 
 constexpr int kKeys = 64;          // keys per tile
 constexpr int kWaveRows = 32;      // query rows per wave
-constexpr int kMaxPages = 2048;    // block-table entries staged in LDS
+constexpr int kMaxPages = 2048;    // block-table entries in LDS at a time
 constexpr int kTileWords = 8;      // int32 words of a tile record
 constexpr float kNegInf = -__builtin_inff();
 // keys of a workgroup's range up to which every 32 keys have an exponent
@@ -127,8 +127,7 @@ __global__ __launch_bounds__(NW * 64, 2) void prefill_attn_kernel(PrefillArgs a)
   const bool paged = a.block_tables != nullptr;
   const int bs_mask = (1 << a.bs_log2) - 1;
   int key_end = min(rec[6], pos0 + nrows);  // (keys past the tile's last row are never attended)
-  if (paged)  // the table's width, and the staged pages
-    key_end = min(key_end, min(a.max_blocks, (key_begin >> a.bs_log2) + kMaxPages) << a.bs_log2);
+  if (paged) key_end = min(key_end, a.max_blocks << a.bs_log2);  // the table's width
   const int64_t tok = (int64_t)a.Hkv * DH; // elements between consecutive keys
 
   // query rows as the B operand of S^T: lane (h, col) holds row col, dims 16 ks + 8 h .. + 7
@@ -143,32 +142,48 @@ __global__ __launch_bounds__(NW * 64, 2) void prefill_attn_kernel(PrefillArgs a)
   const int pos_first = pos0 + r0;           // of the wave's first row
   const int pos_last = min(pos_first + kWaveRows - 1, pos0 + nrows - 1);
 
-  const int pg0 = key_begin >> a.bs_log2;    // first page staged
+  // Block-table entries in LDS: entry i from the first page on at slot i mod
+  // kMaxPages, the first kMaxPages here, the rest half a ring at a time once
+  // the loop has left the half they replace.
+  const int pg0 = key_begin >> a.bs_log2;
+  const int npg = ((key_end + bs_mask) >> a.bs_log2) - pg0;
+  const int32_t* bt = paged ? a.block_tables + (int64_t)seq * a.max_blocks + pg0 : nullptr;
+  int staged = kMaxPages;
   if (paged) {
     if (tid == 0) {
       lds.holes = 0;
-      lds.first = kMaxPages;
+      lds.first = 0x7fffffff;
     }
     __syncthreads();
-    const int npg = ((key_end + bs_mask) >> a.bs_log2) - pg0;
-    const int32_t* bt = a.block_tables + (int64_t)seq * a.max_blocks + pg0;
     for (int i = tid; i < npg; i += NT) {
       const int p = bt[i];
-      lds.pages[i] = p;
+      if (i < kMaxPages) lds.pages[i] = p;
       if (p < 0) lds.holes = 1;
     }
     __syncthreads();
   }
+  auto page = [&](int key) { return lds.pages[((key >> a.bs_log2) - pg0) & (kMaxPages - 1)]; };
+  // the ring's next half, at the start of key tile n0's step (by every wave;
+  // the waves a step behind still read tile n0 - kKeys, the loads ahead reach
+  // 4 tiles, 256 pages at most, past that one: its first use is behind the
+  // step's barrier)
+  auto turn_pages = [&](int n0) {
+    if (!paged || staged >= npg) return;  // uniform
+    const int low = (max(n0 - kKeys, key_begin) >> a.bs_log2) - pg0;
+    if (low < staged - kMaxPages / 2) return;  // uniform
+    const int end = min(staged + kMaxPages / 2, npg);
+    for (int i = staged + tid; i < end; i += NT) lds.pages[i & (kMaxPages - 1)] = bt[i];
+    staged += kMaxPages / 2;
+  };
   const bool holes = paged && __builtin_amdgcn_readfirstlane(lds.holes) != 0;
   int64_t spare = 0;  // the row an unmapped key reads instead (of a key that exists; its weight is zero)
   if (holes) {        // uniform
-    const int npg = ((key_end + bs_mask) >> a.bs_log2) - pg0;
     for (int i = tid; i < npg; i += NT)
-      if (lds.pages[i] >= 0) atomicMin(&lds.first, i);
+      if (bt[i] >= 0) atomicMin(&lds.first, i);
     __syncthreads();
     const int first = __builtin_amdgcn_readfirstlane(lds.first);
-    if (first == kMaxPages) key_end = key_begin;  // no key at all
-    else spare = (int64_t)lds.pages[first] << a.bs_log2;
+    if (first >= npg) key_end = key_begin;  // no key at all
+    else spare = (int64_t)bt[first] << a.bs_log2;
   }
 
   // K/V rows of a tile go from memory straight to LDS (no registers, no LDS
@@ -192,7 +207,7 @@ __global__ __launch_bounds__(NW * 64, 2) void prefill_attn_kernel(PrefillArgs a)
       const int kc = min(n0 + r, key_end - 1);
       int64_t row = kv0 + kc;
       if (paged) {
-        const int p = lds.pages[(kc >> a.bs_log2) - pg0];
+        const int p = page(kc);
         row = p >= 0 ? ((int64_t)p << a.bs_log2) + (kc & bs_mask) : spare;
       }
       const int64_t off = row * tok + hk * DH;
@@ -264,7 +279,7 @@ __global__ __launch_bounds__(NW * 64, 2) void prefill_attn_kernel(PrefillArgs a)
     }
     if (holes) {  // uniform
       const int key = min(n0 + lane, key_end - 1);
-      const uint64_t mapped = __ballot(lds.pages[(key >> a.bs_log2) - pg0] >= 0) >> (4 * h);
+      const uint64_t mapped = __ballot(page(key) >= 0) >> (4 * h);
 #pragma unroll
       for (int t = 0; t < 2; ++t)
 #pragma unroll
@@ -390,6 +405,7 @@ __global__ __launch_bounds__(NW * 64, 2) void prefill_attn_kernel(PrefillArgs a)
     if (!SKEW || w < NW / 2) {
       for (int n0 = key_begin; n0 <= last; n0 += kKeys) {
         const int nf = n0 + DIST * kKeys;
+        turn_pages(n0);
         if (nf <= last) issue(kf, vf, nf);
         scores(kb, n0);
         values(vb, n0);
@@ -401,6 +417,7 @@ __global__ __launch_bounds__(NW * 64, 2) void prefill_attn_kernel(PrefillArgs a)
       int vp = 0;
       for (int n0 = key_begin; n0 <= last; n0 += kKeys) {
         const int nf = n0 + DIST * kKeys;
+        turn_pages(n0);
         if (nf <= last) issue(kf, vf, nf);
         if (n0 > key_begin) values(vp, n0 - kKeys);
         scores(kb, n0);
@@ -542,14 +559,12 @@ Tiling make_tiles(const int64_t* ql, const int64_t* kl, int n, int H, int Hkv, i
   }
   const int64_t units = H / hw;  // workgroups per tile
   const int64_t target = std::max<int64_t>(4, (keys * units * 2 + 3 * cus - 1) / (3 * cus));
-  const int64_t most = std::max<int64_t>(1, (int64_t)(kMaxPages - 1) * block_size / kKeys);  // a part's pages fit LDS
   t.tiles.reserve(tiles);
   int64_t q0 = 0, k0 = 0;
   for (int b = 0; b < n; ++b) {
     for (int64_t r = 0; r < ql[b]; r += t.rows) {
       const int64_t nr = std::min<int64_t>(t.rows, ql[b] - r), pos = kl[b] - ql[b] + r, end = pos + nr, nt = key_tiles(end);
       int64_t parts = tiles * units <= cus && 2 * nt > 3 * target ? (nt + target - 1) / target : 1;
-      if (block_size > 0) parts = std::max(parts, (nt + most - 1) / most);
       const int64_t per = (nt + parts - 1) / parts;
       parts = (nt + per - 1) / per;
       if (parts > 1) t.merges.push_back({t.slots, (int32_t)parts, (int32_t)(q0 + r), (int32_t)nr});

@@ -1,7 +1,9 @@
 """The prefill attention kernel against the fp64 oracle at the edges of its
 tiles: rows around 1, a wave and a tile, keys around a key tile, every head
-group form, both head sizes, pages from one token on, unmapped pages, tiles
-cut over keys, and both workgroup sizes."""
+group form, both head sizes, pages from one token on, unmapped pages, and each
+form of the kernel: 4 and 8 waves, whole tiles and tiles cut over keys, paged
+and contiguous K/V, block tables longer than LDS holds (each case names the
+form it takes)."""
 
 import numpy as np
 import pytest
@@ -57,6 +59,61 @@ def test_both_workgroup_sizes_and_cuts_are_reached():
             for H, Hkv, _, ql, kl, page in CASES}
     assert rows == {128, 256}
     assert [prefill_tiles(ql, kl, H, Hkv, page, 256)[3] > 0 for H, Hkv, _, ql, kl, page in CASES][-2:] == [True, True]
+
+
+def make_plan(ql, kl, H, Hkv, page, cus):
+    """A plan for a device of ``cus`` compute units (1: no tile is cut)."""
+    plan = PrefillPlan(ql, kl, H, Hkv, page, torch.device("cuda"))
+    tiles, merges, plan.tile_rows, plan.slots = prefill_tiles(ql, kl, H, Hkv, page, cus)
+    plan.ntiles, plan.nmerges = len(tiles), len(merges)
+    plan.work = torch.from_numpy(np.concatenate([tiles.ravel(), merges.ravel()])).cuda()
+    return plan
+
+
+FORMS = [
+    # waves, heads per workgroup, cut, heads, kv heads, head dim, new rows, keys, page (None: contiguous), unmapped pages
+    (8, 2, False, 2, 1, 128, [300, 5], [1800, 2100], 16, []),
+    (8, 2, True, 2, 1, 128, [300, 5], [1800, 2100], 16, [(0, 0), (1, 77)]),
+    (8, 2, False, 4, 1, 64, [129, 2], [2000, 1537], 32, [(0, 5), (1, 48)]),
+    (8, 2, True, 2, 1, 64, [40], [4136], 64, []),
+    (8, 1, False, 3, 1, 128, [257], [1900], 16, [(0, 0), (0, 118)]),
+    (8, 1, True, 3, 1, 64, [31], [1600], 16, []),
+    (8, 2, False, 2, 1, 128, [3150], [3150], None, []),
+    (8, 1, False, 1, 1, 64, [3300], [3300], None, []),
+    (8, 2, True, 2, 1, 64, [3200], [3200], None, []),
+    (4, 2, True, 2, 1, 128, [700], [700], None, []),
+    (4, 1, False, 3, 1, 64, [129, 70], [129, 70], None, []),
+    # block tables of more entries than LDS holds: two and more turns of the ring
+    (8, 2, False, 2, 1, 64, [70], [4700], 1, [(0, 10), (0, 3000), (0, 4699)]),
+    (8, 1, False, 1, 1, 128, [33], [3200], 1, [(0, n) for n in range(2100)]),  # the first mapped page past the first turn
+    (8, 2, True, 2, 1, 128, [5], [5001], 1, [(0, 4000)]),
+    (8, 2, False, 2, 1, 128, [70], [9001], 2, []),
+    (4, 2, False, 2, 1, 64, [1, 1, 1], [3000, 64, 65], 1, [(0, 2500)]),
+    (4, 1, False, 1, 1, 128, [3, 1, 1], [2600, 64, 65], 1, []),
+]
+
+
+@pytest.mark.parametrize("form", range(len(FORMS)))
+def test_every_form_matches_oracle(form):
+    waves, hw, cut, H, Hkv, D, ql, kl, page, unmapped = FORMS[form]
+    print(f"case: prefill attention form {FORMS[form][:9]}", flush=True)
+    plan = make_plan(ql, kl, H, Hkv, page, 256 if cut else 1)
+    assert (plan.tile_rows * hw // 32, 2 if H // Hkv % 2 == 0 else 1, plan.slots > 0) == (waves, hw, cut)
+    vb = synth.verify_batch(90 + form, kl, ql, num_heads=H, num_kv_heads=Hkv, head_dim=D, block_size=page or 16)
+    bt = vb.block_tables.copy()
+    for b, i in unmapped:
+        bt[b, i] = -1
+    f = lambda x: torch.from_numpy(np.ascontiguousarray(x, dtype=np.float32)).cuda().bfloat16()  # noqa: E731
+    k, v = vb.k_cache, vb.v_cache
+    if page is None:
+        k, v = (np.concatenate([c[[p for p in bt[b] if p >= 0]].reshape(-1, Hkv, D)[:n] for b, n in enumerate(kl)])
+                for c in (k, v))
+    out = prefill_attention(f(vb.q), f(k), f(v), plan, 1 / np.sqrt(D), D,
+                            None if page is None else torch.from_numpy(bt).cuda())
+    torch.cuda.synchronize()
+    want = ora.verify_attention(vb.q, vb.k_cache, vb.v_cache, bt, vb.context_lens, vb.cu_seqlens_q, vb.positions,
+                                1 / np.sqrt(D), H, Hkv)
+    assert_close(out, want, "bf16", f"form {FORMS[form][:9]}")
 
 
 def test_prefill_attention_refuses_bad_shapes():

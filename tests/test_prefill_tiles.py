@@ -23,8 +23,6 @@ def test_tiles_cover_every_pair_once(heads, block_size, ql, kl):
         first = row0 - q0[seq]
         assert 0 <= first and first + nr <= ql[seq] and pos == kl[seq] - ql[seq] + first
         assert kv0 == (k0[seq] if block_size is None else 0)
-        if block_size is not None:
-            assert -(-end // block_size) - begin // block_size <= 2048
         for r in range(nr):
             seen[row0 + r, begin:min(end, pos + r + 1)] += 1
         parts.setdefault((row0, nr), []).append((begin, end, slot))
@@ -47,3 +45,16 @@ def test_bad_lengths_are_refused():
     for ql, kl in (([0], [4]), ([5], [4]), ([4, 4], [4])):
         with pytest.raises(ValueError):
             prefill_tiles(ql, kl, 16, 8, 256, 256)
+
+
+@pytest.mark.parametrize("heads", [(16, 8), (32, 8), (64, 8), (8, 8), (3, 1), (2, 1)])
+@pytest.mark.parametrize("block_size", [1, 16, 256])
+def test_partials_are_bounded(heads, block_size):
+    # only a step whose tiles leave compute units idle is cut over keys (into
+    # parts of two thirds of a compute unit's share of its key tiles or more),
+    # whatever the page size: its partials stay within 2.5 workgroups' rows a
+    # compute unit, 85 MB at 256
+    for ql, kl in (([32000], [32000]), ([40000], [40000]), ([1], [40000]), ([300, 5], [20000, 33000]), ([128] * 8, [9000] * 8)):
+        tiles, merges, rows, slots = prefill_tiles(ql, kl, *heads, block_size, 256)
+        assert slots * heads[0] * rows * (128 + 2) * 4 <= 2.5 * 256 * 256 * (128 + 2) * 4, (ql, kl, slots)
+    assert prefill_tiles([40000], [40000], *heads, 1, 256)[3] == prefill_tiles([40000], [40000], *heads, 256, 256)[3]
