@@ -197,7 +197,7 @@ __global__ __launch_bounds__(NW * 64, 2) void prefill_attn_kernel(PrefillArgs a)
   // waits below and the barriers order them.)
   auto load_lds = [&](const bf16_t* src, unsigned char* dst) {
     const uint32_t at = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)dst);
-    __asm__ volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(at), "v"(src) : "memory");
+    __asm__ volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(at), "v"(src) : "memory", "m0");
   };
   auto issue = [&](int kb, int vb, int n0) {
 #pragma unroll
