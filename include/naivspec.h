@@ -137,8 +137,9 @@ int nsv_prefill_tiles(const int64_t* seqlens_q, const int64_t* seqlens_k,
  * Load-only measurement kernels, no reference counterpart (the ceilings
  * against which bench.py --ceiling reads the verify-attention kernels).
  * nsv_verify_attention_load_floor reads exactly the K/V bytes of a bf16,
- * D = 128 verify-attention call over `splits` key splits per (sequence, kv
- * head), in the key-split kernel's access pattern, and computes nothing;
+ * D = 128 verify-attention call planned with `splits` key splits per
+ * (sequence, kv head), in the key-split kernel's access pattern (each context
+ * cut as that kernel cuts it), and computes nothing;
  * nsv_stream_read reads `bytes` (a multiple of 16) of contiguous memory in
  * `workgroups` equal chunks.  `sink` is a device buffer of one uint32 per
  * workgroup that is written only for an improbable checksum.
@@ -189,14 +190,16 @@ int nsv_verify_attention_noalloc(void* out, const void* q, const void* k_cache,
 int nsv_stamp_configure(void* buf, int calls);
 
 /* The kernel nsv_verify_attention runs for these arguments on a device
- * with `cus` compute units (cus <= 0: the current device) and the key
- * splits per sequence it cuts (1: none).  Host-only query, launches
+ * with `cus` compute units (cus <= 0: the current device) and the most key
+ * splits it cuts a sequence into (1: none); the key-split kernel counts each
+ * context's own by its length, never more than these (kv_split_tokens 0), as
+ * the others leave splits past a context's end out.  Host-only query, launches
  * nothing; no reference counterpart (it exposes this library's plan for
  * tests and tuning).  Returns what nsv_verify_attention would return for
  * the shape (0, or the rejection code). */
 #define NSV_ATTN_DSLICED 0   /* bf16, workgroup = (pair, head-dim slice) */
 #define NSV_ATTN_KEY_SPLIT 1 /* bf16, workgroup = (pair, key split)      */
-#define NSV_ATTN_F32 2       /* fp32, VALU dot products                  */
+#define NSV_ATTN_F32 2       /* fp32, fp32 matrix instruction            */
 int nsv_verify_attention_plan(int B, int H, int Hkv, int D, int block_size,
                               int max_blocks, int max_q_len, int dtype,
                               int kv_split_tokens, int cus, int* kernel,

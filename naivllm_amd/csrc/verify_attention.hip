@@ -2017,8 +2017,10 @@ int make_plan(int B, int H, int Hkv, int D, int block_size, int max_blocks, int 
   const bool ks_wins = kv_split_tokens > 0 || pairs * 16 >= ks_slots || max_ctx >= 4096 || p->MT == 1;
   if (dtype == NSV_BF16 && ks_fits && ks_wins) {
     // key-split kernel: each sequence's keys evenly over about CUs / pairs
-    // splits (none when the pairs alone cover the chip), but no split
-    // shorter than 160 keys (shorter splits pay the merge for too few loads:
+    // splits (none when the pairs alone cover the chip), but no split of a
+    // context as long as the table shorter than 160 keys (shorter contexts
+    // take fewer splits, split_len_ks, which may be shorter; shorter splits
+    // pay the merge for too few loads:
     // at 8 pairs x 1.25k keys, 8 splits take 11.5 us, 10 12.7, 16 12.7; at
     // 32 pairs 8 take 13.3 against 14.4 for 5), or the caller's fixed split
     // length
@@ -2149,7 +2151,8 @@ void launch_f32(const VerifyArgs& a, int D, dim3 grid, hipStream_t s) {
 // ---------------------------------------------------------------------------
 // attn_load_floor_kernel reads exactly the K/V bytes of the key-split kernel,
 // in its access pattern: workgroup = (pair, key split) with every split of a
-// pair on one XCD, the block-table row staged in LDS first, then each of the
+// pair on one XCD and the splits counted by each context (as for more than one
+// 16-row tile of query rows), the block-table row staged in LDS first, then each of the
 // 8 waves streams its interleaved 16-key tiles (K and V rows of one kv head,
 // whole 256-byte rows, 4 + 4 loads of 16 bytes per lane) with one tile in
 // flight.  Nothing is computed; the loaded words are folded into one value
@@ -2165,9 +2168,10 @@ __global__ __launch_bounds__(512) void attn_load_floor_kernel(VerifyArgs a, uint
   for (int j = threadIdx.x; j < a.max_blocks; j += 512) pages[j] = a.block_tables[(int64_t)b * a.max_blocks + j];
   const int ctx = context_len(a, b);
   __syncthreads();
-  const int nsplit = num_splits(a, ctx);
+  bool fine;  // (no part in the loads)
+  const int len = ctx < (1 << 22) ? split_len_ks<2>(a, ctx, fine) : split_len(a, ctx);
+  const int nsplit = (ctx + len - 1) / len;
   if (split >= nsplit) return;
-  const int len = split_len(a, ctx);
   const int kb = split * len, ke = min(ctx, kb + len);
   const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int ntiles = (ke - kb + 15) / 16;
