@@ -21,13 +21,13 @@
 //
 // Measured on MI355X (the verify kernel on causal blocks of 64 / G rows,
 // which every prefill ran on before -> this kernel): 8 prompts of ~1000
-// tokens, 16/8 heads, 538 -> 59 us (557 TFLOP/s); prompts of 2900 and 4050
-// tokens behind 4096 cached keys, 32/8 heads, 5283 -> 725 us (924); 8192
-// tokens, 32/8 heads, 535 us (1028); one prompt of 1206 tokens, 16/8 heads,
-// 85 -> 31 us.  With K/V staged through registers instead of straight to LDS
-// and both waves of a SIMD in step: 59-64, 781-793, 590 and 31 us (counters:
-// matrix cores and VALU 42% busy each, nearly one after the other; 34% of the
-// wave cycles waiting).
+// tokens, 16/8 heads, 538 -> 69 us (475 TFLOP/s); prompts of 2900 and 4050
+// tokens behind 4096 cached keys, 32/8 heads, 5283 -> 790-815 us (820-850);
+// 8192 tokens, 32/8 heads, 600 us (916); one prompt of 1206 tokens, 16/8
+// heads, 85 -> 32 us.  What the parts of it gave was measured with an exponent
+// reference moved lazily, which is less precise (see there): these four 59,
+// 725, 535 and 31 us; with K/V staged through registers instead of straight to
+// LDS and both waves of a SIMD in step 59-64, 781-793, 590 and 31.
 
 #include "common.h"
 
@@ -294,11 +294,13 @@ __global__ __launch_bounds__(NW * 64, 2) void prefill_attn_kernel(PrefillArgs a)
     // scores, in 1e-5 (the verify kernel on causal blocks; one reference,
     // moved lazily -> these): one prompt of 1,206 tokens 193; 204 -> 192, 40
     // rows behind 256 keys 203; 229 -> 203, 900 behind 2,048 216; 231 -> 205.
-    // The rescaling costs up to 14% of the time (2,900 and 4,050 rows of 32/8
-    // heads behind 4,096 keys 721 -> 822 us, 8,192 tokens 538 -> 600, one
-    // prompt of 1,206 33 -> 34).  A reference every 64 keys from the first key
-    // on takes 33 us there, but is 1 to 3% further off than the verify kernel
-    // (1,206 tokens 196, 40 rows behind 256 keys 209).
+    // The rescaling costs up to 8% of the time (lazily moved -> these, 2,900
+    // and 4,050 rows of 32/8 heads behind 4,096 keys 730 -> 790 us, 8,192
+    // tokens 552 -> 595, one prompt of 1,206 32 -> 33.5), and 4% more where the
+    // second reference is moved between the products instead of before them.
+    // Not precise enough: a reference every 64 keys from the first key on
+    // (1,206 tokens 196, 40 rows behind 256 keys 209), every 128 keys past the
+    // first 256 (4,050 rows behind 4,096 keys 221; the verify kernel 220).
     const bool fine = n0 < key_begin + kFineKeys;  // uniform
     float mx[2];
 #pragma unroll
@@ -314,7 +316,6 @@ __global__ __launch_bounds__(NW * 64, 2) void prefill_attn_kernel(PrefillArgs a)
       const bool on = m > kNegInf && !((m_run - m) * sc > kRefDrop);
       const float alpha = on ? __builtin_amdgcn_exp2f((m_ref - m) * sc) : 1.f;  // (from -inf: 0)
       m_ref = on ? m : m_ref;
-      l_run *= alpha;
       return alpha;
     };
     auto rescale = [&](float alpha) {
@@ -324,8 +325,15 @@ __global__ __launch_bounds__(NW * 64, 2) void prefill_attn_kernel(PrefillArgs a)
 #pragma unroll
         for (int i = 0; i < 16; ++i) acc[dt][i] *= alpha;
     };
-    rescale(move(mx[0]));
-    float nb = m_ref == kNegInf ? 0.f : -m_ref * sc;
+    const float alpha0 = move(mx[0]);
+    const float nb0 = m_ref == kNegInf ? 0.f : -m_ref * sc;
+    float alpha1 = 1.f, nb1 = nb0;  // of the tile's second 32 keys
+    if (fine) {  // uniform
+      alpha1 = move(half_max(mx[1]));
+      nb1 = m_ref == kNegInf ? 0.f : -m_ref * sc;
+    }
+    rescale(alpha0);
+    l_run *= alpha0;
     // O^T += V^T P^T, 16 keys per step: element j of lane half h is key
     // 8 (j / 4) + 4 h + j % 4 of the step in both operands.  A step's weights
     // are computed, and its V operands read, during the step before's products.
@@ -349,26 +357,20 @@ __global__ __launch_bounds__(NW * 64, 2) void prefill_attn_kernel(PrefillArgs a)
       float sum = 0.f;
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        const float p0 = __builtin_amdgcn_exp2f(fmaf(s[st >> 1][(st & 1) * 8 + 2 * e], sc, nb));
-        const float p1 = __builtin_amdgcn_exp2f(fmaf(s[st >> 1][(st & 1) * 8 + 2 * e + 1], sc, nb));
+        const float p0 = __builtin_amdgcn_exp2f(fmaf(s[st >> 1][(st & 1) * 8 + 2 * e], sc, st < ST / 2 ? nb0 : nb1));
+        const float p1 = __builtin_amdgcn_exp2f(fmaf(s[st >> 1][(st & 1) * 8 + 2 * e + 1], sc, st < ST / 2 ? nb0 : nb1));
         sum += p0 + p1;
         pw[e] = pack_bf16x2(p0, p1);
       }
-      l_run += sum;
+      l_run = st == ST / 2 ? fmaf(l_run, alpha1, sum) : l_run + sum;
       pB[st & 1] = as_bf16x8(pw);
     };
     read(0);
     weights(0);
 #pragma unroll
     for (int st = 0; st < ST; ++st) {
-      const bool second = fine && st + 1 == ST / 2;  // the second 32 keys come next
-      float alpha = 1.f;
       if (st + 1 < ST) {
         read(st + 1);
-        if (second) {  // uniform
-          alpha = move(half_max(mx[1]));
-          nb = m_ref == kNegInf ? 0.f : -m_ref * sc;
-        }
         weights(st + 1);
       }
 #pragma unroll
@@ -376,7 +378,7 @@ __global__ __launch_bounds__(NW * 64, 2) void prefill_attn_kernel(PrefillArgs a)
         const uint2 lo = va[st & 1][dt][0], hi = va[st & 1][dt][1];
         acc[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_bf16x8(u32x4{lo.x, lo.y, hi.x, hi.y}), pB[st & 1], acc[dt], 0, 0, 0);
       }
-      if (second) rescale(alpha);
+      if (st + 1 == ST / 2 && fine) rescale(alpha1);
       __builtin_amdgcn_sched_barrier(0);
     }
   };
@@ -518,17 +520,18 @@ __global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillMergeArgs a) 
 // (two query heads of a kv head where the group is even) reads a K/V tile for
 // twice the rows of a 4-wave one, but fewer, larger workgroups fill the chip
 // worse and idle longer at the causal edge.  Measured on MI355X, 4 against 8
-// waves: 8 prompts of ~1000 tokens (16/8 heads) 59 against 70 us, one of 1206
-// 36 against 40, 4096 (32/8 heads) 171 against 148, two of 2900-4050 behind
-// 4096 cached keys 800 against 725: 8 waves from 24 key tiles per tile on
-// average.
+// waves: 8 prompts of 1000 tokens (16/8 heads) 69 against 66 us, one of 1206
+// 32 against 34; 32/8 heads: 1206 42 against 47, 2048 70 against 74, 3000 111
+// against 112, 4096 194 against 172, two of 2900-4050 behind 4096 cached keys
+// 833 against 814: 8 waves from 24 key tiles per tile on average.
 //
 // Cut over keys: where the tiles alone are fewer than the compute units, a
-// tile's chain of key tiles (~1.8 us each with one wave per SIMD) is the
+// tile's chain of key tiles (~2 us each with one wave per SIMD) is the
 // call's time, so tiles longer than 1.5 targets are cut into parts of about
 // `target` key tiles and merged by a second kernel: 40 rows behind 4096 keys
-// 114 -> 20 us (targets 3 and 4; 6: 21, 8: 24), 270 rows of 32/8 heads 120 ->
-// 50-62 (16, 12), one prompt of 1206 40 -> 31 (4; 3: 35, 8: 34).  With more
+// 130 -> 22 us, 270 rows of 32/8 heads 141 -> 60, one prompt of 1206 40 -> 32
+// (other targets, with a lazily moved reference: 20 us at 3 and 4, 21 at 6, 24
+// at 8; 50-62 at 16 and 12; 31 at 4, 35 at 3, 34 at 8).  With more
 // tiles than compute units the partials cost what the shorter chain saves
 // (1206 of 32/8 heads, 304 workgroups: 41.7 -> 39-43; 8 prompts 59 ->
 // 64-172), so those stay whole.
