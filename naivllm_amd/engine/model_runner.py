@@ -52,8 +52,8 @@ class ModelRunner:
         self._inputs = torch.zeros(n64 + (max_num_sequences * max_blocks + 1) // 2, **i64)
         self.verify_vars = {"k": k, **self._views(self._inputs, rows, max_num_sequences, max_blocks),
                             "logits": torch.empty(rows, model.cfg.vocab_size, dtype=model.dtype, device=dev)}
-        self._staging = [torch.zeros(self._inputs.shape, dtype=torch.int64, pin_memory=dev.type == "cuda")
-                         for _ in range(STAGING)]
+        # (one pinned allocation for all of them: each takes ~0.5 ms)
+        self._staging = torch.zeros(STAGING, self._inputs.numel(), dtype=torch.int64, pin_memory=dev.type == "cuda")
         self._staged = [{name: t.numpy() for name, t in self._views(h, rows, max_num_sequences, max_blocks).items()}
                         for h in self._staging]
         for h in self._staged:  # inert rows until a call fills them
