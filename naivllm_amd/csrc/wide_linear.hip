@@ -305,7 +305,12 @@ struct WidePlan {
 };
 
 // Plain: the largest even split of the reduction's 256-element chunks that
-// keeps one workgroup per CU and at least two chunks each: 64-column
+// keeps one workgroup per CU and at least two chunks each, or, where the even
+// ones leave more than a third of those workgroups unused, an uneven one (an
+// odd range costs a chunk of zeros; a whole layer at 72 rows, even only -> so,
+// us: 4096 x 11008, 43 chunks, 1 -> 8 splits 224 -> 146, library 171; 3584 x
+// 18944, 74 chunks, 2 -> 9 splits 223 -> 169, library 235; 2560 x 9728, 38
+// chunks, 2 -> 12 splits 148 -> 122, library 133): 64-column
 // workgroups while that leaves at most four chunks (the columns alone are
 // few, so each CU reads little of x), 128-column ones beyond (half the
 // workgroups read x, twice the splits).  MI355X, 72 rows, graph-replayed over
@@ -333,17 +338,18 @@ WidePlan wide_plan(int M, int N, int K, int epi, bool packed, int cus) {
   }
   if (packed) return {128, K == 1024 || K == 2048 || K == 4096 ? 1 : 0};  // the packed layout's reductions
   const int nck = K / kWlKC;
-  auto even = [&](int cols) {
+  auto cut = [&](int cols) {
     const int groups = (N + cols - 1) / cols;
     int s = cus / groups;
     s = s > nck / 2 ? nck / 2 : s;
-    for (s = s < 1 ? 1 : s; nck % s; --s) {
+    const int most = s < 1 ? 1 : s;
+    for (s = most; nck % s; --s) {
     }
-    return s;
+    return 3 * s < 2 * most ? most : s;
   };
-  const int s64 = even(64);
+  const int s64 = cut(64);
   if (nck / s64 <= 4) return {64, s64};
-  return {128, even(128)};
+  return {128, cut(128)};
 }
 
 int wide_cus() {

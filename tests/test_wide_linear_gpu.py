@@ -42,6 +42,19 @@ def test_wide_linear_plain(M, N, K):
         assert y.isnan().all()  # the consumer sums the partials; y is not touched
 
 
+# reductions of 11 and 38 chunks, which no even split cuts finely enough: 64
+# columns (ranges of 2 and 3 chunks) and 128 columns (3 and 4)
+@pytest.mark.parametrize("M", [1, 17, 128])
+@pytest.mark.parametrize("N,K,splits", [(1040, 2816, 5), (2560, 9728, 12)])
+def test_wide_linear_uneven_splits(M, N, K, splits):
+    assert qm.wide_splits(M, N, K) == splits
+    print(f"case: wide linear M={M} N={N} K={K} uneven splits={splits}", flush=True)
+    x, w = randn(M + N, M, K), randn(K + 1, N, K, scale=K ** -0.5)
+    part = torch.full((splits, M, N), float("nan"), device="cuda")
+    qm.wide_linear(x, w, None, part)
+    torch.testing.assert_close(part.double().sum(0), product(x, w), **BF16)
+
+
 def test_wide_linear_plan_covers_its_forms():
     assert [qm.wide_splits(72, N, K) for N, K in ((1040, 256), (1040, 2048), (8208, 2560), (33024, 1280))] == [1, 4, 2, 1]
     assert qm.wide_splits(129, 1024, 1024) == qm.wide_splits(8, 1024, 1000) == qm.wide_splits(8, 1000, 1024) == 0
