@@ -12,8 +12,8 @@ pre-attention epilogue (q/k RMSNorm + RoPE + paged KV store), verify
 attention, o_proj (with the residual add as its epilogue), gate_up
 (post-attention RMSNorm prologue, SiLU * up epilogue) and down (residual
 add epilogue).  Up to WIDE_ROWS rows they run on the weight-streaming
-projections (8 launches per layer), wider batches on hipBLASLt between this
-library's residual-RMSNorm, epilogue, attention and SiLU kernels.  The LM
+projections where the hidden size is above WIDE_HIDDEN (8 launches per
+layer), other batches on hipBLASLt between this library's residual-RMSNorm, epilogue, attention and SiLU kernels.  The LM
 head runs on this library's streaming kernel up to lm_head_rows() rows (79 at
 hidden 1024, 19 at hidden 4096: the activations staged in one CU's LDS), from
 a copy of its weight packed in that kernel's load order, on the
@@ -262,8 +262,12 @@ def silu_mul(gate_up: torch.Tensor, out: torch.Tensor) -> None:
 # so its cost grows with rows x hidden size, while hipBLASLt's wide tiles
 # reuse the activations.  Measured on MI355X (each projection alone): at
 # hidden 1024 the fused layer (4 launches) beats hipBLASLt + the separate
-# norm / SiLU kernels up to 72 rows (38 vs 42 us per layer at 72); at hidden
-# 4096 the fused kernel wins at 9 rows and loses from about 16.
+# norm / SiLU kernels up to 72 rows (38 vs 42 us per layer at 72; attention
+# included and graph-replayed, 65 vs 72 at 72, 66 vs 72 at 80, 84 vs 73 at 96);
+# at hidden 4096 it wins at 9 rows and loses from about 20 (graph-replayed
+# against the weight-streaming kernel: 93 vs 108 at 13, 96 vs 109 at 16, 116 vs
+# 116 at 20, 148 vs 124 at 36): the line, at the drafts + 1 rows of one request,
+# is on the safe side of that.
 FUSED_ROWS = 80
 FUSED_ROWS_WIDE = 12  # hidden size above 2048
 
@@ -274,8 +278,19 @@ FUSED_ROWS_WIDE = 12  # hidden size above 2048
 # Measured on MI355X at hidden 4096, graph-replayed over rotating weights, the
 # library against it: 72 rows qkv 23.1 -> 17.0 us, o 16.2 -> 11.5, gate_up with
 # SiLU 53.5 + 4 -> 46, down 42.9 -> 25.5, LM head 283 -> 239; 108 rows 23.7 ->
-# 21.2, 16.4 -> 14.1, 55 + 4 -> 55, 43.1 -> 30.6, 291 -> 282.
+# 21.2, 16.4 -> 14.1, 55 + 4 -> 55, 43.1 -> 30.6, 291 -> 282.  A whole layer at
+# 16, 36, 72, 96 and 128 rows: 126 -> 116, 146 -> 128, 178 -> 150, 198 -> 164,
+# 225 -> 187 us (intermediate size 14336: 145 -> 143, 158 -> 157, 191 -> 185,
+# 128 rows 244 -> 197, but 54 rows 164 -> 168).  The LM head alone at hidden
+# 1024, 2048 and 4096: 80 rows 84 -> 66, 161 -> 121, 272 -> 241, 128 rows 90 ->
+# 79, 167 -> 143, 279 -> 277.
 WIDE_ROWS = 128
+# Hidden size past which the layers do (the head at any): up to it the fused
+# kernel serves 80 rows, and past those a layer takes, library against this
+# kernel, at hidden 1024 72.7 -> 73.7 us (88 rows), 79.3 -> 84.7 (108), 81.5 ->
+# 89.8 (128), at 2048 103.5 -> 101.2 (96), 109.3 -> 111.0 (108), 114 -> 117
+# (128); at 2560 72 rows 132 -> 122, 128 rows 185 -> 154.
+WIDE_HIDDEN = 2048
 
 
 # Rows up to which the LM head runs on this library's kernels: nsv_linear
@@ -363,11 +378,10 @@ class Qwen3Verify:
         # count, so its rows come out the same at every batch shape)
         self.decode_linears = False
 
-
     def pack_lm_head(self) -> None:
         """Repack the LM head's weight in the streaming kernel's load order
-        (nsv_lm_head_pack) where this shape streams; the row-major weight
-        stays for the embedding lookup and for more rows than that.  Called
+        (nsv_lm_head_pack) where this shape streams; it serves up to WIDE_ROWS
+        rows, the row-major weight the embedding lookup and more rows.  Called
         once by the constructor; whoever replaces or edits self.lm_head
         afterwards calls it again."""
         self.lm_head_packed = None
@@ -387,7 +401,7 @@ class Qwen3Verify:
         cfg = self.cfg
         E, I, HD = cfg.hidden_size, cfg.intermediate_size, cfg.num_heads * cfg.head_dim
         # (its loads take weights on 16 bytes: a view at an odd offset stays on hipBLASLt)
-        if T > WIDE_ROWS or E % 4 or E > 4096 or not all(
+        if T > WIDE_ROWS or E <= WIDE_HIDDEN or E % 4 or E > 4096 or not all(
                 L[k].is_contiguous() and L[k].data_ptr() % 16 == 0
                 for L in self.layers for k in ("qkv", "o", "gate_up", "down")):
             return None

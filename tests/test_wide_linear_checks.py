@@ -77,3 +77,12 @@ def test_shapes_past_32_bit_offsets_are_not_taken(M, N, K, taken):
 
 def test_packed_takes_the_packed_layouts_reductions():
     assert [qm.wide_splits(80, 1024, K, packed=True) for K in (512, 1024, 2048, 3072, 4096, 5120)] == [0, 1, 1, 0, 1, 0]
+
+
+@pytest.mark.parametrize("hidden,rows,taken", [(1024, 81, False), (2048, 128, False), (2304, 13, True), (2304, 128, True),
+                                               (2304, 129, False), (4096, 128, True)])
+def test_layers_take_the_kernel_where_it_is_faster(hidden, rows, taken):
+    # (up to hidden 2048 the library is, past the rows of the fused kernel)
+    cfg = qm.Qwen3Config(vocab_size=64, hidden_size=hidden, num_layers=1, num_heads=2, num_kv_heads=1, head_dim=128,
+                         intermediate_size=256, max_position=64)
+    assert (qm.Qwen3Verify(cfg, "cpu")._wide_splits(rows) is not None) is taken
