@@ -1241,8 +1241,8 @@ __global__ __launch_bounds__(NW * 64, 8 / NW) void verify_attn_ks_kernel(VerifyA
       mx = row_max4(mx);
       const float m_old = m_run[mt];
       // the rule's two inputs, ready before the scores: what the reference
-      // does not go below, and how far down (log2 domain; up if negative) it
-      // has to move at least
+      // does not go below, and the distance down (log2 domain; up if negative)
+      // below which it moves
       const float least = fine ? kNegInf : m_old;
       const float drop = fine ? (float)max(kRefDropExp - __builtin_amdgcn_frexp_expf(l_run[mt]), 0) : -kRefSlack;
       const float m_new = fmaxf(least, mx);
