@@ -11,15 +11,15 @@ layer: the QKV projection (with the input RMSNorm as its prologue), the
 pre-attention epilogue (q/k RMSNorm + RoPE + paged KV store), verify
 attention, o_proj (with the residual add as its epilogue), gate_up
 (post-attention RMSNorm prologue, SiLU * up epilogue) and down (residual
-add epilogue).  Up to WIDE_ROWS rows they run on the weight-streaming
-projections where the hidden size is above WIDE_HIDDEN (8 launches per
-layer), other batches on hipBLASLt between this library's residual-RMSNorm, epilogue, attention and SiLU kernels.  The LM
-head runs on this library's streaming kernel up to lm_head_rows() rows (79 at
-hidden 1024, 19 at hidden 4096: the activations staged in one CU's LDS), from
-a copy of its weight packed in that kernel's load order, on the
-weight-streaming kernel from the same copy up to WIDE_ROWS, and on hipBLASLt
-beyond.  Weights are random (seeded): no checkpoint is
-loaded.
+add epilogue). Up to WIDE_ROWS rows they run on the weight-streaming
+projections where the hidden size is above WIDE_HIDDEN (8 launches per layer),
+other batches on hipBLASLt between this library's residual-RMSNorm, epilogue,
+attention and SiLU kernels. The LM head runs on this library's streaming kernel
+up to lm_head_rows() rows (79 at hidden 1024, 19 at hidden 4096: the
+activations staged in one CU's LDS), from a copy of its weight packed in that
+kernel's load order, on the weight-streaming kernel from the same copy up to
+WIDE_ROWS, and on hipBLASLt beyond. Weights are random (seeded): no checkpoint
+is loaded.
 
 The forward takes the verify metadata explicitly (positions, slots, block
 tables, context lengths, cu_seqlens) so a whole forward is capturable in a
