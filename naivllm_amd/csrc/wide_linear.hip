@@ -325,7 +325,10 @@ struct WidePlan {
 // columns), else three per workgroup (24576 x 4096, 72 rows: 46 us for 256
 // workgroups, 52 with four slots, 58 with one; the library GEMM alone 53.5,
 // its SiLU kernel 4 more), or four past 80 rows, whose registers three slots
-// of two waves do not hold (108 rows: 54.7 against 74.4).
+// of two waves do not hold (108 rows: 54.7 against 74.4), and wherever three
+// would leave a second turn of a few workgroups and four do not (intermediate
+// size 14336, 299 or 224 workgroups, a whole layer with three -> four: 16 rows
+// 137 -> 127 us, 54 167 -> 148, 72 184 -> 163, the library 143, 163 and 189).
 WidePlan wide_plan(int M, int N, int K, int epi, bool packed, int cus) {
   if (M <= 0 || M > kWlMaxRows || N <= 0 || K <= 0 || N % 16 || K % kWlKC) return {0, 0};
   // byte offsets into the weight and into the activations' padded row tiles fit an int
@@ -334,7 +337,9 @@ WidePlan wide_plan(int M, int N, int K, int epi, bool packed, int cus) {
   if (epi == 1) {
     if (N % 32 || packed) return {0, 0};
     if (N / 32 <= cus) return {16, 1};
-    return {M <= 80 ? 48 : 64, 1};
+    const int tiles = N / 32;
+    const bool one_turn = (tiles + 2) / 3 <= cus || (tiles + 3) / 4 > cus;  // of 48 columns, or none of 64
+    return {M <= 80 && one_turn ? 48 : 64, 1};
   }
   if (packed) return {128, K == 1024 || K == 2048 || K == 4096 ? 1 : 0};  // the packed layout's reductions
   const int nck = K / kWlKC;

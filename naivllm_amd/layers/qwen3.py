@@ -280,10 +280,10 @@ FUSED_ROWS_WIDE = 12  # hidden size above 2048
 # SiLU 53.5 + 4 -> 46, down 42.9 -> 25.5, LM head 283 -> 239; 108 rows 23.7 ->
 # 21.2, 16.4 -> 14.1, 55 + 4 -> 55, 43.1 -> 30.6, 291 -> 282.  A whole layer at
 # 16, 36, 72, 96 and 128 rows: 126 -> 116, 146 -> 128, 178 -> 150, 198 -> 164,
-# 225 -> 187 us (intermediate size 14336: 145 -> 143, 158 -> 157, 191 -> 185,
-# 128 rows 244 -> 197, but 54 rows 164 -> 168).  The LM head alone at hidden
-# 1024, 2048 and 4096: 80 rows 84 -> 66, 161 -> 121, 272 -> 241, 128 rows 90 ->
-# 79, 167 -> 143, 279 -> 277.
+# 225 -> 187 us (intermediate size 14336: 143 -> 127, 157 -> 141, 189 -> 163,
+# 128 rows 244 -> 197; 16384: 54 rows 171 -> 163, 16 rows 146 -> 149).  The LM
+# head alone at hidden 1024, 2048 and 4096: 80 rows 84 -> 66, 161 -> 121, 272 ->
+# 241, 128 rows 90 -> 79, 167 -> 143, 279 -> 277.
 WIDE_ROWS = 128
 # Hidden size past which the layers do (the head at any): up to it the fused
 # kernel serves 80 rows, and past those a layer takes, library against this

@@ -72,6 +72,19 @@ def test_wide_linear_swiglu(M, I, K):
     torch.testing.assert_close(y.float(), F.silu(gu[:, :I]) * gu[:, I:], **BF16)
 
 
+# 48 columns would take a second turn of workgroups and 64 do not (769 and 1024
+# slots of 16), or both do (1025)
+@pytest.mark.parametrize("M", [1, 80])
+@pytest.mark.parametrize("I", [12304, 16384, 16400])
+def test_wide_linear_swiglu_turns(M, I):
+    print(f"case: wide linear swiglu M={M} I={I}", flush=True)
+    x, w = randn(M + I, M, 256), randn(3, 2 * I, 256, scale=1 / 16)
+    y = torch.full((M, I), float("nan"), dtype=torch.bfloat16, device="cuda")
+    qm.wide_linear(x, w, y, swiglu=True)
+    gu = product(x, w).to(torch.bfloat16).float()
+    torch.testing.assert_close(y.float(), F.silu(gu[:, :I]) * gu[:, I:], **BF16)
+
+
 @pytest.mark.parametrize("M", [2, 20, 72, 100, 128])
 @pytest.mark.parametrize("N,K", [(160, 1024), (32976, 1024), (33088, 2048)])
 def test_wide_linear_packed(M, N, K):
