@@ -37,6 +37,9 @@ SIGNATURES: dict[str, tuple] = {
     "nsv_verify_attention": (
         _c_int,
         [_c_vp] * 8 + [_c_f32] + [_c_int] * 10 + [_c_vp, _c_size, _c_vp]),
+    "nsv_verify_attention_tile_refs": (
+        _c_int,
+        [_c_vp] * 8 + [_c_f32] + [_c_int] * 10 + [_c_vp, _c_size, _c_vp]),
     "nsv_verify_attention_noalloc_max_scratch": (_c_size, []),
     "nsv_verify_attention_noalloc": (
         _c_int,

@@ -954,7 +954,9 @@ __global__ __launch_bounds__(kBf16Waves * 64, 1) void verify_attn_bf16_kernel(Ve
 // at slot X ^ (r % VCH)) into the operand layout; a CU ingests whole rows
 // several times faster than the operand order's 64 bytes from each of 16
 // keys (config 4 on MI355X: 369 -> 356 us per call).
-template <int MT, int DH, int NW, bool WROW = (NSV_KS_WROW != 0)>
+// TILE_REFS: exponent references follow every tile whatever the splits (an
+// argument for it would cost every other call ~0.1 us).
+template <int MT, int DH, int NW, bool TILE_REFS = false, bool WROW = (NSV_KS_WROW != 0)>
 __global__ __launch_bounds__(NW * 64, 8 / NW) void verify_attn_ks_kernel(VerifyArgs a) {
   constexpr int NT = NW * 64;
   constexpr int TK = 16;          // keys per wave tile
@@ -1036,6 +1038,7 @@ __global__ __launch_bounds__(NW * 64, 8 / NW) void verify_attn_ks_kernel(VerifyA
   const int qlen = q1 - q0;
   bool fine;
   const int len = split_len_ks<MT>(a, ctx, fine);
+  if (TILE_REFS) fine = true;
   const int nsplit = num_splits_ks(ctx, len);
   if (split >= nsplit || qlen < 0) return;  // uniform per workgroup
   const int kb = split * len;
@@ -2110,17 +2113,19 @@ void launch_bf16_dc(const VerifyArgs& a, dim3 grid, hipStream_t s) {
     hipLaunchKernelGGL((verify_attn_bf16_kernel<MT, DH, DC, false, bf16_stages(MT, DH, DC, false)>), grid, dim3(kBf16Waves * 64), 0, s, a);
 }
 
-template <int MT>
-int launch_ks(const VerifyArgs& a, int D, dim3 grid, hipStream_t s) {
-  if constexpr (MT <= 3) {
-    constexpr int NW = kKsWaves;
-    if (D == 128)
-      hipLaunchKernelGGL((verify_attn_ks_kernel<MT, 128, NW>), grid, dim3(NW * 64), 0, s, a);
-    else
-      hipLaunchKernelGGL((verify_attn_ks_kernel<MT, 64, NW>), grid, dim3(NW * 64), 0, s, a);
-    return NSV_OK;
-  }
-  return NSV_ERR_UNSUPPORTED;
+template <int MT, bool TILE_REFS>
+void launch_ks(const VerifyArgs& a, int D, dim3 grid, hipStream_t s) {
+  constexpr int NW = kKsWaves;
+  if (D == 128)
+    hipLaunchKernelGGL((verify_attn_ks_kernel<MT, 128, NW, TILE_REFS>), grid, dim3(NW * 64), 0, s, a);
+  else
+    hipLaunchKernelGGL((verify_attn_ks_kernel<MT, 64, NW, TILE_REFS>), grid, dim3(NW * 64), 0, s, a);
+}
+template <bool TILE_REFS>
+void launch_ks(const VerifyArgs& a, int MT, int D, dim3 grid, hipStream_t s) {  // (the plan: MT <= 3)
+  if (MT == 1) launch_ks<1, TILE_REFS>(a, D, grid, s);
+  else if (MT == 2) launch_ks<2, TILE_REFS>(a, D, grid, s);
+  else launch_ks<3, TILE_REFS>(a, D, grid, s);
 }
 
 // Head-dim slice width dc = D / dqc must be one the kernels are built for
@@ -2271,17 +2276,13 @@ int scratch_for_current_device(hipStream_t stream, void** out) {
 // The kernels of one verify-attention launch (the head subset a.g0 ..
 // a.g0 + a.G - 1 of every kv head): the key-split kernel, or the d-sliced /
 // fp32 kernel and, with key splits, the merge kernel.
-int launch_verify(const VerifyArgs& a, const Plan& p, int D, int dtype, hipStream_t s) {
+int launch_verify(const VerifyArgs& a, const Plan& p, int D, int dtype, bool tile_refs, hipStream_t s) {
   int rc = NSV_OK;
   const dim3 grid(8 * p.S * a.P8 * p.dqc);
   if (dtype == NSV_BF16 && p.ks) {
     const dim3 kgrid(8 * a.P8, p.S);  // (pair, split)
-    switch (p.MT) {
-      case 1: rc = launch_ks<1>(a, D, kgrid, s); break;
-      case 2: rc = launch_ks<2>(a, D, kgrid, s); break;
-      default: rc = launch_ks<3>(a, D, kgrid, s); break;
-    }
-    if (rc != NSV_OK) return rc;
+    if (tile_refs) launch_ks<true>(a, p.MT, D, kgrid, s);
+    else launch_ks<false>(a, p.MT, D, kgrid, s);
   } else if (dtype == NSV_BF16) {
     const dim3 dgrid(8 * a.P8, p.dqc, p.S);  // (pair, head-dim slice, split)
     switch (p.MT) {
@@ -2369,11 +2370,11 @@ int nsv_verify_attention_plan(int B, int H, int Hkv, int D, int block_size, int 
   return NSV_OK;
 }
 
-int nsv_verify_attention(void* out, const void* q, const void* k_cache, const void* v_cache,
-                         const int32_t* block_tables, const int64_t* context_lens, const int32_t* cu_seqlens_q,
-                         const int64_t* positions, float scale, int B, int T, int H, int Hkv, int D, int block_size,
-                         int max_blocks, int max_q_len, int dtype, int kv_split_tokens, void* workspace,
-                         size_t workspace_bytes, void* stream) {
+static int verify_attention(void* out, const void* q, const void* k_cache, const void* v_cache,
+                            const int32_t* block_tables, const int64_t* context_lens, const int32_t* cu_seqlens_q,
+                            const int64_t* positions, float scale, int B, int T, int H, int Hkv, int D, int block_size,
+                            int max_blocks, int max_q_len, int dtype, int kv_split_tokens, void* workspace,
+                            size_t workspace_bytes, bool tile_refs, void* stream) {
   Plan p;
   int rc = make_plan(B, H, Hkv, D, block_size, max_blocks, max_q_len, dtype, kv_split_tokens, device_cus(), &p);
   if (rc != NSV_OK) return rc;
@@ -2426,10 +2427,30 @@ int nsv_verify_attention(void* out, const void* q, const void* k_cache, const vo
     if (g_stamp_buf && 8 * p.S * a.P8 * p.dqc <= kStampMaxWgs)
       a.stamps = g_stamp_buf + (size_t)(g_stamp_next++ % (unsigned)g_stamp_calls) * kStampMaxWgs * kStampSlots;
 #endif
-    rc = launch_verify(a, p, D, dtype, s);
+    rc = launch_verify(a, p, D, dtype, tile_refs, s);
     if (rc != NSV_OK) return rc;
   }
   return NSV_OK;
+}
+
+int nsv_verify_attention(void* out, const void* q, const void* k_cache, const void* v_cache,
+                         const int32_t* block_tables, const int64_t* context_lens, const int32_t* cu_seqlens_q,
+                         const int64_t* positions, float scale, int B, int T, int H, int Hkv, int D, int block_size,
+                         int max_blocks, int max_q_len, int dtype, int kv_split_tokens, void* workspace,
+                         size_t workspace_bytes, void* stream) {
+  return verify_attention(out, q, k_cache, v_cache, block_tables, context_lens, cu_seqlens_q, positions, scale, B, T, H,
+                          Hkv, D, block_size, max_blocks, max_q_len, dtype, kv_split_tokens, workspace, workspace_bytes,
+                          false, stream);
+}
+
+int nsv_verify_attention_tile_refs(void* out, const void* q, const void* k_cache, const void* v_cache,
+                                   const int32_t* block_tables, const int64_t* context_lens,
+                                   const int32_t* cu_seqlens_q, const int64_t* positions, float scale, int B, int T,
+                                   int H, int Hkv, int D, int block_size, int max_blocks, int max_q_len, int dtype,
+                                   int kv_split_tokens, void* workspace, size_t workspace_bytes, void* stream) {
+  return verify_attention(out, q, k_cache, v_cache, block_tables, context_lens, cu_seqlens_q, positions, scale, B, T, H,
+                          Hkv, D, block_size, max_blocks, max_q_len, dtype, kv_split_tokens, workspace, workspace_bytes,
+                          true, stream);
 }
 
 int nsv_verify_attention_load_floor(const void* k_cache, const void* v_cache, const int32_t* block_tables,

@@ -85,6 +85,7 @@ def paged_attention_verify(
     kv_split_tokens: int = 0,
     out: torch.Tensor | None = None,
     allocation_free: bool = False,
+    tile_references: bool = False,
 ) -> torch.Tensor:
     """Verify a chunk of drafted tokens against the paged KV cache.
 
@@ -99,7 +100,9 @@ def paged_attention_verify(
     (a preallocated result) and ``allocation_free`` (run through
     nsv_verify_attention_noalloc: the library's fixed per-device scratch
     instead of a workspace, ``out`` required, index tensors already int32 /
-    int64 and contiguous, so the call allocates nothing).  Rows at position
+    int64 and contiguous, so the call allocates nothing), ``tile_references``
+    (an exponent reference per tile of keys, nsv_verify_attention_tile_refs;
+    not with allocation_free).  Rows at position
     -1 come back as zeros (the reference leaves them meaningless; nothing
     reads them).
     """
@@ -130,6 +133,8 @@ def paged_attention_verify(
     if allocation_free:
         if out is None:
             raise ValueError("allocation_free=True needs a preallocated out")
+        if tile_references:
+            raise ValueError("allocation_free=True takes no tile_references")
         rc = h.nsv_verify_attention_noalloc(
             out.data_ptr(), query.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), block_tables.data_ptr(),
             context_lens.data_ptr(), cu_seqlens_q.data_ptr(), positions.data_ptr(), float(scale), batch_size,
@@ -143,7 +148,7 @@ def paged_attention_verify(
         batch_size, num_heads, num_kv_heads, head_dim, block_size, max_num_blocks, qlen_bound, code,
         kv_split_tokens))
     ws = _lib.workspace(query.device, ws_bytes, "verify_attention")
-    rc = h.nsv_verify_attention(
+    rc = (h.nsv_verify_attention_tile_refs if tile_references else h.nsv_verify_attention)(
         out.data_ptr(), query.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(),
         block_tables.data_ptr(), context_lens.data_ptr(), cu_seqlens_q.data_ptr(), positions.data_ptr(),
         float(scale), batch_size, query.shape[0], num_heads, num_kv_heads, head_dim, block_size,
@@ -185,17 +190,23 @@ def store_kvcache(
     _lib.check(rc, "store_kvcache")
 
 
-def _prefill_work(seqlens_q, seqlens_k, num_heads: int, num_kv_heads: int, block_size: int | None, cus: int,
-                  pinned: bool) -> tuple[torch.Tensor, list[int]]:
-    """nsv_prefill_tiles into a host tensor; returns (its words, [tiles,
-    merges, tile_rows, slots])."""
+def _prefill_lengths(seqlens_q, seqlens_k) -> tuple[list[int], list[int]]:
+    """The lengths as lists of ints, checked."""
     seqlens_q, seqlens_k = [int(x) for x in seqlens_q], [int(x) for x in seqlens_k]
-    n = len(seqlens_q)
-    if n != len(seqlens_k):
+    if len(seqlens_q) != len(seqlens_k):
         raise ValueError("seqlens_q and seqlens_k differ in length")
     for i, (ql, kl) in enumerate(zip(seqlens_q, seqlens_k)):
         if not 0 < ql <= kl:
             raise ValueError(f"prefill sequence {i}: {ql} query rows over {kl} keys")
+    return seqlens_q, seqlens_k
+
+
+def _prefill_work(seqlens_q, seqlens_k, num_heads: int, num_kv_heads: int, block_size: int | None, cus: int,
+                  pinned: bool) -> tuple[torch.Tensor, list[int]]:
+    """nsv_prefill_tiles into a host tensor; returns (its words, [tiles,
+    merges, tile_rows, slots])."""
+    seqlens_q, seqlens_k = _prefill_lengths(seqlens_q, seqlens_k)
+    n = len(seqlens_q)
     q, k, counts = (ctypes.c_int64 * n)(*seqlens_q), (ctypes.c_int64 * n)(*seqlens_k), (ctypes.c_int32 * 4)()
     words = 4096
     while True:
@@ -219,20 +230,13 @@ def prefill_tiles(seqlens_q, seqlens_k, num_heads: int, num_kv_heads: int, block
     return work[:8 * nt].view(nt, 8).numpy(), work[8 * nt:].view(nm, 4).numpy(), rows, slots
 
 
-class PrefillPlan:
-    """The work list of one prefill step on the device, in one transfer.
+class _StepList:
+    """A prefill step's metadata on the device, in one transfer (``work``).
 
     The transfer is enqueued on the stream that is current here and not waited
     for; a call on another stream waits for it on the device (use_on)."""
 
-    def __init__(self, seqlens_q, seqlens_k, num_heads: int, num_kv_heads: int, block_size: int | None, device):
-        cus = torch.cuda.get_device_properties(device).multi_processor_count
-        # (as _lib.upload: not waited for, except inside a capture, which refuses the wait)
-        ahead = not torch.cuda.is_current_stream_capturing()
-        work, (self.ntiles, self.nmerges, self.tile_rows, self.slots) = _prefill_work(
-            seqlens_q, seqlens_k, num_heads, num_kv_heads, block_size, cus, ahead)
-        self.num_heads, self.num_kv_heads, self.block_size = num_heads, num_kv_heads, block_size
-        self.sequences, self.rows, self.keys = len(seqlens_q), int(sum(seqlens_q)), int(sum(seqlens_k))
+    def _send(self, work: torch.Tensor, device, ahead: bool) -> None:
         self.work = work.to(device, non_blocking=ahead)
         stream = torch.cuda.current_stream(device)
         self.stream = stream.cuda_stream
@@ -251,6 +255,73 @@ class PrefillPlan:
         if self.ready is not None:
             stream.wait_event(self.ready)
         self.work.record_stream(stream)
+
+
+def _send_ahead() -> bool:
+    """As _lib.upload: a step's transfer is not waited for, except inside a
+    capture, which refuses the wait."""
+    return not torch.cuda.is_current_stream_capturing()
+
+
+class PrefillPlan(_StepList):
+    """The prefill kernel's work list of one step on the device."""
+
+    def __init__(self, seqlens_q, seqlens_k, num_heads: int, num_kv_heads: int, block_size: int | None, device):
+        cus = torch.cuda.get_device_properties(device).multi_processor_count
+        ahead = _send_ahead()
+        work, (self.ntiles, self.nmerges, self.tile_rows, self.slots) = _prefill_work(
+            seqlens_q, seqlens_k, num_heads, num_kv_heads, block_size, cus, ahead)
+        self.num_heads, self.num_kv_heads, self.block_size = num_heads, num_kv_heads, block_size
+        self.sequences, self.rows, self.keys = len(seqlens_q), int(sum(seqlens_q)), int(sum(seqlens_k))
+        self._send(work, device, ahead)
+
+
+class PrefillRows(_StepList):
+    """The verify kernel's metadata of a prefill step of a few rows per
+    sequence (verify_serves_prefill) on the device: context_lens, positions
+    and cu_seqlens_q, one entry per sequence or row."""
+
+    def __init__(self, seqlens_q, seqlens_k, device):
+        ql, kl = _prefill_lengths(seqlens_q, seqlens_k)
+        n, rows, ahead = len(ql), sum(ql), _send_ahead()
+        work = torch.empty(n + rows + n // 2 + 1, dtype=torch.int64, pin_memory=ahead)
+        work[:n] = torch.tensor(kl, dtype=torch.int64)
+        work[n:n + rows] = torch.cat([torch.arange(k - q, k) for q, k in zip(ql, kl)])
+        work[n + rows:].view(torch.int32)[:n + 1] = torch.tensor([0] + ql).cumsum(0)
+        self.sequences, self.rows, self.max_q_len = n, rows, max(ql)
+        self._send(work, device, ahead)
+        self.context_lens, self.positions = self.work[:n], self.work[n:n + rows]
+        self.cu_seqlens_q = self.work[n + rows:].view(torch.int32)[:n + 1]
+
+
+def verify_serves_prefill(seqlens_q, seqlens_k, num_heads: int, num_kv_heads: int, block_size: int,
+                          max_num_blocks: int) -> bool:
+    """Whether a paged bf16 prefill step runs on the verify kernel, one block
+    of rows per sequence, and not on the prefill kernel.
+
+    The prefill kernel's waves hold 32 rows of one query head and a workgroup
+    two heads of a kv head, so a short suffix behind a long prefix leaves most
+    of its waves without rows and a group of 4 or more heads reads its K/V
+    twice or more; the verify kernel packs the group's rows.  MI355X,
+    graph-replayed, prefill -> verify kernel, us per layer: 16/8 heads, one
+    sequence of 9 rows behind 1,024 keys 14.7 -> 8.8, behind 16,384 47 -> 28,
+    eight of 24 behind 4,096 61 -> 30; 32/8 heads, eight of 4 behind 4,096 98 ->
+    26, of 12 99 -> 31.  The lines: up to 48 packed rows (the key-split kernel's
+    three row tiles) wherever that kernel takes the table and 8 pairs or more
+    are there, beyond one row tile (2 pairs and 16 rows of 3 heads: 17 -> 22);
+    where it does not take the table (24,000 keys in pages of one or 16 tokens)
+    groups of more than two heads only (32/8 heads 524 -> 342, 16/8 274 -> 336).
+    Up to 64 packed rows (the verify kernel's most) groups of more than two
+    heads with 1,536 keys or more: 32/8 heads, eight of 16 rows behind 4,096
+    keys 101 -> 77, behind 1,024 24 -> 27; 16/8 heads, of 32 63 -> 77."""
+    group, pairs, longest = num_heads // num_kv_heads, len(seqlens_q) * num_kv_heads, max(seqlens_k, default=0)
+    rows = group * max(seqlens_q, default=0)
+    if rows < 1 or rows > 64 or max_num_blocks * block_size >= 1 << 22:
+        return False
+    key_split = block_size >= 16 and max_num_blocks <= 1024
+    if rows <= 48:
+        return (pairs >= 8 or rows <= 16) and (key_split or group > 2)
+    return pairs >= 8 and key_split and group > 2 and longest >= 1536
 
 
 def _aligned(t: torch.Tensor) -> torch.Tensor:
@@ -368,8 +439,9 @@ class Attention(nn.Module):
         the step's own K/V already stored in it, as the reference's
         paged_attention_prefill (:328-363); without, from the step's
         contiguous K/V, as its varlen flash path (:257-325).  bf16 runs on
-        the prefill kernel (``prefill_attention``), fp32 on the verify kernel
-        over causal blocks of rows (``_prefill_rows``);
+        the prefill kernel (``prefill_attention``), paged steps of a few rows
+        per sequence on the verify kernel (``verify_serves_prefill``), fp32 on
+        the verify kernel over causal blocks of rows (``_prefill_rows``);
       * decode (neither flag): one query row per sequence attending its
         whole context (:759-767), served by the same verify kernel with
         each row at position context_lens - 1."""
@@ -385,14 +457,18 @@ class Attention(nn.Module):
         self.k_cache = self.v_cache = torch.tensor([])
 
     def _prefill_bf16(self, context, q, k, v, scale: float) -> torch.Tensor:
-        """The prefill branch on the prefill kernel; the step's work list is
-        built by its first layer and kept with the step's Context."""
+        """The prefill branch on the prefill kernel, or on the verify kernel
+        for a few rows per sequence; the step's work list is built by its
+        first layer and kept with the step's Context."""
         paged = context.block_tables is not None
         if context.seqlens_q is None or context.seqlens_k is None:
             raise ValueError("a prefill step needs context.seqlens_q and context.seqlens_k")
         bs = self.block_size if paged else None
         key = (self.num_heads, self.num_kv_heads, bs, q.device)
         plans = context.__dict__.setdefault("prefill_plans", {})
+        if paged and verify_serves_prefill(context.seqlens_q, context.seqlens_k, self.num_heads, self.num_kv_heads, bs,
+                                           context.block_tables.shape[1]):
+            return self._prefill_few(context, plans, q, scale)
         plan = plans.get(key)
         if plan is None:
             plan = plans[key] = PrefillPlan(context.seqlens_q, context.seqlens_k, self.num_heads, self.num_kv_heads,
@@ -402,6 +478,22 @@ class Attention(nn.Module):
                                      context.block_tables.to(q.device))
         return prefill_attention(q, k.reshape(-1, self.num_kv_heads, self.head_dim),
                                  v.reshape(-1, self.num_kv_heads, self.head_dim), plan, scale, self.head_dim)
+
+    def _prefill_few(self, context, plans: dict, q, scale: float) -> torch.Tensor:
+        """A paged prefill step of a few rows per sequence as one verify call."""
+        rows = plans.get(q.device)
+        if rows is None:
+            rows = plans[q.device] = PrefillRows(context.seqlens_q, context.seqlens_k, q.device)
+        if q.shape[0] < rows.rows:
+            raise ValueError(f"query must have at least {rows.rows} rows, got {q.shape[0]}")
+        tables = context.block_tables.to(q.device)
+        if tables.shape[0] < rows.sequences:
+            raise ValueError(f"{rows.sequences} sequences but {tables.shape[0]} block-table rows")
+        rows.use_on(torch.cuda.current_stream(q.device))
+        return paged_attention_verify(
+            q, self.k_cache, self.v_cache, tables[:rows.sequences], rows.context_lens, rows.cu_seqlens_q, rows.positions,
+            scale, self.num_heads, self.num_kv_heads, self.head_dim, self.block_size, 64, max_q_len=rows.max_q_len,
+            tile_references=True)
 
     def forward(self, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor) -> torch.Tensor:
         context = get_context()

@@ -36,7 +36,8 @@ import torch
 import torch.nn.functional as F
 
 from naivllm_amd import _lib
-from naivllm_amd.layers.attention import PrefillPlan, paged_attention_verify, prefill_attention
+from naivllm_amd.layers.attention import (PrefillPlan, PrefillRows, paged_attention_verify, prefill_attention,
+                                          verify_serves_prefill)
 
 
 @dataclass
@@ -420,9 +421,14 @@ class Qwen3Verify:
         *per_row, last, bt, new, lens = prefill_rows(token_lists, starts, tables, bs)
         rows = _lib.upload(np.concatenate([*per_row, last]), self.device)
         T = sum(new)
-        plan = PrefillPlan(new, lens, self.cfg.num_heads, self.cfg.num_kv_heads, bs, self.device)
-        return self.forward(rows[:T], rows[T:2 * T], rows[2 * T:3 * T], _lib.upload(bt, self.device), None, None, 0,
-                            logits_rows=rows[3 * T:], prefill=plan)
+        H, Hkv = self.cfg.num_heads, self.cfg.num_kv_heads
+        args = (rows[:T], rows[T:2 * T], rows[2 * T:3 * T], _lib.upload(bt, self.device))
+        if verify_serves_prefill(new, lens, H, Hkv, bs, bt.shape[1]):
+            few = PrefillRows(new, lens, self.device)
+            return self.forward(*args, few.context_lens, few.cu_seqlens_q, few.max_q_len, logits_rows=rows[3 * T:],
+                                tile_references=True)
+        plan = PrefillPlan(new, lens, H, Hkv, bs, self.device)
+        return self.forward(*args, None, None, 0, logits_rows=rows[3 * T:], prefill=plan)
 
     def allocate_kv_cache(self, num_blocks: int, block_size: int) -> None:
         """One [num_blocks, block_size, Hkv, D] K and V pool per layer
@@ -436,13 +442,15 @@ class Qwen3Verify:
     def forward(self, input_ids: torch.Tensor, positions: torch.Tensor, slot_mapping: torch.Tensor,
                 block_tables: torch.Tensor, context_lens: torch.Tensor, cu_seqlens_q: torch.Tensor,
                 max_q_len: int, logits_out: torch.Tensor | None = None,
-                logits_rows: torch.Tensor | None = None, prefill: PrefillPlan | None = None) -> torch.Tensor:
+                logits_rows: torch.Tensor | None = None, prefill: PrefillPlan | None = None,
+                tile_references: bool = False) -> torch.Tensor:
         """Verify forward over T = sum of per-sequence query rows.  Rows at
         position -1 are inert padding (no KV store, zero attention output).
         Returns logits [T, vocab] (written into logits_out when given), or
         only the rows ``logits_rows`` indexes (the prefill's last rows).
         prefill: the rows are whole prompts' (block_tables then one row per
-        prompt; context_lens, cu_seqlens_q and max_q_len are not used)."""
+        prompt; context_lens, cu_seqlens_q and max_q_len are not used).
+        tile_references: as paged_attention_verify's."""
         if self.dtype != torch.bfloat16:
             raise ValueError("the fused forward kernels are bf16")
         cfg = self.cfg
@@ -460,7 +468,7 @@ class Qwen3Verify:
             block_m = max(16, 1 << (max_q_len - 1).bit_length())
             attn = lambda li: paged_attention_verify(  # noqa: E731
                 q, self.k_caches[li], self.v_caches[li], block_tables, context_lens, cu_seqlens_q, positions,
-                self.scale, H, Hkv, D, self.block_size, block_m, max_q_len=max_q_len)
+                self.scale, H, Hkv, D, self.block_size, block_m, max_q_len=max_q_len, tile_references=tile_references)
         # embedding lookup, layer 0's input norm, and the rotary rows of the step's
         # positions (gathered once for every layer, so that each layer's epilogue
         # loads them without first loading the positions) in one launch

@@ -8,6 +8,7 @@ import numpy as np
 import pytest
 import torch
 
+import naivllm_amd.layers.attention as at
 from naivllm_amd.layers.attention import Attention
 from naivllm_amd.utils import synth
 from naivllm_amd.utils.context import get_context, reset_context, set_context
@@ -158,3 +159,49 @@ def test_prefill_step_through_set_context_contiguous(dtype):
                                          np.array([n]), np.array([0, n], np.int32), np.arange(n),
                                          1 / np.sqrt(D), H, Hkv))
     assert_close(out.view(-1, H, D), np.concatenate(want), dtype, "varlen prefill via set_context")
+
+
+# packed rows around the verify kernel's row tiles (48 of 8 pairs; 16 of
+# fewer), pages it takes and does not, with a page missing, a table row for a
+# sequence that is not in the step, and columns past the longest context
+FEW = [
+    # heads, kv heads, page, new rows, keys, on the verify kernel
+    (16, 8, 64, [24], [300], True),
+    (16, 8, 64, [25], [300], False),
+    (16, 8, 16, [1, 24, 7], [1, 2000, 7], True),
+    (32, 8, 256, [12], [1700], True),
+    (32, 8, 256, [13], [1700], True),
+    (32, 8, 256, [16, 2], [1536, 1000], True),
+    (32, 8, 256, [16, 2], [1535, 1000], False),
+    (8, 2, 16, [4, 1], [200, 90], True),
+    (8, 2, 16, [5, 1], [200, 90], False),
+    (16, 8, 8, [3], [700], False),
+    (32, 8, 8, [3], [700], True),
+    (6, 2, 16, [5, 5, 5, 16], [64, 65, 5, 400], True),
+]
+
+
+@pytest.mark.parametrize("case", range(len(FEW)))
+def test_prefill_of_few_rows_matches_oracle(case, monkeypatch):
+    H, Hkv, page, ql, kl, few = FEW[case]
+    print(f"case: prefill step of few rows {FEW[case]}", flush=True)
+    vb = synth.verify_batch(50 + case, kl, ql, num_heads=H, num_kv_heads=Hkv, block_size=page)
+    bt = np.pad(vb.block_tables, ((0, 1), (0, 2)), constant_values=-1)
+    if kl[0] > 2 * page:
+        bt[0, 1] = -1
+    layer, f = _layer(vb)
+    calls = []
+    real = at.prefill_attention
+    monkeypatch.setattr(at, "prefill_attention", lambda *a: calls.append(1) or real(*a))
+    set_context(True, cu_seqlens_q=torch.from_numpy(vb.cu_seqlens_q).cuda(), slot_mapping=None,
+                block_tables=torch.from_numpy(bt).cuda(), seqlens_q=ql, seqlens_k=kl)
+    z = torch.zeros(sum(ql), Hkv, vb.head_dim, device="cuda", dtype=torch.bfloat16)
+    try:
+        outs = [layer(f(vb.q), z, z) for _ in range(2)]  # (the second layer of a step finds its rows kept)
+        torch.cuda.synchronize()
+    finally:
+        reset_context()
+    assert (not calls) is few and torch.equal(*outs)
+    want = ora.verify_attention(vb.q, vb.k_cache, vb.v_cache, bt[:-1], vb.context_lens, vb.cu_seqlens_q, vb.positions,
+                                1 / np.sqrt(vb.head_dim), H, Hkv)
+    assert_close(outs[0].view(-1, H, vb.head_dim), want, "bf16", f"few rows {FEW[case]}")

@@ -151,3 +151,18 @@ def test_prefill_matches_dense_forward():
     want = torch.stack([dense_forward(model, torch.tensor(t, device="cuda"))[-1] for t in toks])
     rel = (got.float() - want).norm(dim=1) / want.norm(dim=1)
     assert rel.max() < 2e-2, rel.tolist()
+
+
+def test_prefill_of_a_short_suffix_matches_dense_forward():
+    # a few new tokens behind prefilled pages, as one verify forward
+    print("case: prefill forward of short suffixes", flush=True)
+    model = Qwen3Verify(TINY, "cuda", seed=6)
+    model.allocate_kv_cache(16, 64)
+    rng = np.random.default_rng(62)
+    toks = [[int(x) for x in rng.integers(0, TINY.vocab_size, n)] for n in (136, 195)]
+    tables = [[3, 1, 7], [5, 0, 4, 9]]
+    model.prefill([toks[0][:128], toks[1][:192]], [0, 0], tables)
+    got = model.prefill(toks, [128, 192], tables)
+    want = torch.stack([dense_forward(model, torch.tensor(t, device="cuda"))[-1] for t in toks])
+    rel = (got.float() - want).norm(dim=1) / want.norm(dim=1)
+    assert rel.max() < 2e-2, rel.tolist()

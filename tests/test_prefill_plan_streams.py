@@ -70,6 +70,23 @@ def test_a_capture_holds_no_outside_event(streams):
     assert other.waits == [] and plan.work.uses == []
 
 
+def test_rows_of_a_step_of_few_and_their_streams(streams, monkeypatch):
+    real = torch.empty
+    monkeypatch.setattr(torch, "empty", lambda *a, pin_memory=False, **k: real(*a, **k))
+    rows, other = at.PrefillRows([3, 1, 2], [10, 1, 2], torch.device("cpu")), Stream("other")
+    assert rows.context_lens.tolist() == [10, 1, 2] and rows.positions.tolist() == [7, 8, 9, 0, 0, 1]
+    assert rows.cu_seqlens_q.tolist() == [0, 3, 4, 6] and rows.cu_seqlens_q.dtype == torch.int32 and rows.max_q_len == 3
+    rows.work = Work()
+    rows.use_on(other)
+    assert other.waits == [rows.ready] and rows.work.uses == [other]
+
+
+@pytest.mark.parametrize("ql,kl", [([0], [4]), ([5], [4]), ([1, 1], [4])])
+def test_rows_of_bad_lengths_are_refused(streams, ql, kl):
+    with pytest.raises(ValueError):
+        at.PrefillRows(ql, kl, torch.device("cpu"))
+
+
 def test_views_at_odd_offsets_are_copied():
     base = torch.arange(4 * 2 * 64 + 8, dtype=torch.bfloat16)
     for off in (0, 8):  # whole 16 bytes

@@ -3,6 +3,7 @@ cached prefix, and the lists that do not belong together, on the CPU."""
 
 import pytest
 
+from naivllm_amd.layers.attention import verify_serves_prefill
 from naivllm_amd.layers.qwen3 import prefill_rows
 
 
@@ -27,3 +28,17 @@ def test_lists_of_different_lengths_are_refused(starts, tables):
 def test_starts_outside_the_sequence_are_refused(start):
     with pytest.raises(ValueError, match="outside"):
         prefill_rows([[1, 2]], [start], [[1]], 4)
+
+
+@pytest.mark.parametrize("new,keys,heads,page,width,taken", [
+    ([24], [300], (16, 8), 16, 19, True), ([25], [4000], (16, 8), 16, 250, False),      # 48 packed rows, 8 pairs
+    ([8], [300], (4, 2), 16, 19, True), ([9], [300], (4, 2), 16, 19, False),            # 16 with fewer pairs
+    ([9] * 4, [300] * 4, (4, 2), 16, 19, True),
+    ([9], [300], (16, 8), 8, 38, False), ([9], [300], (32, 8), 8, 38, True),            # pages the key-split kernel does not take
+    ([9], [300], (16, 8), 16, 1024, True), ([9], [300], (16, 8), 16, 1025, False),      # its longest table
+    ([16], [1536], (32, 8), 256, 6, True), ([16], [1535], (32, 8), 256, 6, False),      # 64 packed rows
+    ([32], [4000], (16, 8), 256, 16, False), ([17], [4000], (32, 8), 256, 16, False),
+    ([1], [1], (80, 1), 256, 1, False), ([4], [4], (32, 8), 1, 1 << 22, False),
+])
+def test_steps_of_few_rows(new, keys, heads, page, width, taken):
+    assert verify_serves_prefill(new, keys, *heads, page, width) is taken
