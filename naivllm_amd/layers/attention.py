@@ -147,13 +147,19 @@ def paged_attention_verify(
     ws_bytes = int(h.nsv_verify_attention_workspace_size(
         batch_size, num_heads, num_kv_heads, head_dim, block_size, max_num_blocks, qlen_bound, code,
         kv_split_tokens))
-    ws = _lib.workspace(query.device, ws_bytes, "verify_attention")
+    stream = _lib.stream_ptr(query.device)
+    name = "verify_attention"
+    if tile_references and not torch.cuda.is_current_stream_capturing():
+        # (prefill steps may run beside another stream's rounds: scratch of
+        # their own per stream, of which torch has a fixed pool)
+        name = f"verify_attention on stream {stream}"
+    ws = _lib.workspace(query.device, ws_bytes, name)
     rc = (h.nsv_verify_attention_tile_refs if tile_references else h.nsv_verify_attention)(
         out.data_ptr(), query.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(),
         block_tables.data_ptr(), context_lens.data_ptr(), cu_seqlens_q.data_ptr(), positions.data_ptr(),
         float(scale), batch_size, query.shape[0], num_heads, num_kv_heads, head_dim, block_size,
         max_num_blocks, qlen_bound, code, kv_split_tokens,
-        _lib.ptr(ws), ws_bytes, _lib.stream_ptr(query.device))
+        _lib.ptr(ws), ws_bytes, stream)
     _lib.check(rc, "paged_attention_verify")
     return out
 

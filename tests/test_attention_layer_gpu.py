@@ -9,6 +9,7 @@ import pytest
 import torch
 
 import naivllm_amd.layers.attention as at
+from naivllm_amd import _lib
 from naivllm_amd.layers.attention import Attention
 from naivllm_amd.utils import synth
 from naivllm_amd.utils.context import get_context, reset_context, set_context
@@ -205,3 +206,29 @@ def test_prefill_of_few_rows_matches_oracle(case, monkeypatch):
     want = ora.verify_attention(vb.q, vb.k_cache, vb.v_cache, bt[:-1], vb.context_lens, vb.cu_seqlens_q, vb.positions,
                                 1 / np.sqrt(vb.head_dim), H, Hkv)
     assert_close(outs[0].view(-1, H, vb.head_dim), want, "bf16", f"few rows {FEW[case]}")
+
+
+def test_prefill_of_few_rows_beside_another_stream():
+    # key splits merged through scratch: steps on two streams and a verify call
+    # keep their own
+    print("case: prefill steps of few rows on two streams", flush=True)
+    vb = synth.verify_batch(70, [4000], [4], num_heads=16, num_kv_heads=8, block_size=64)
+    layer, f = _layer(vb)
+    q, z = f(vb.q), torch.zeros(4, 8, vb.head_dim, device="cuda", dtype=torch.bfloat16)
+    set_context(True, cu_seqlens_q=torch.from_numpy(vb.cu_seqlens_q).cuda(), slot_mapping=None,
+                block_tables=torch.from_numpy(vb.block_tables).cuda(), seqlens_q=[4], seqlens_k=[4000])
+    try:
+        want = layer(q, z, z)
+        torch.cuda.synchronize()
+        side = torch.cuda.Stream()
+        got = []
+        for _ in range(8):
+            got.append(layer(q, z, z))
+            with torch.cuda.stream(side):
+                got.append(layer(q, z, z))
+        torch.cuda.synchronize()
+    finally:
+        reset_context()
+    assert all(torch.equal(g, want) for g in got)
+    names = {n for _, _, n in _lib._workspaces}
+    assert {f"verify_attention on stream {s.cuda_stream}" for s in (torch.cuda.current_stream(), side)} <= names
